@@ -500,24 +500,51 @@ static int launch_mmq(GemvArgs a, int KS, hipStream_t s) {
   return launched("mmq");
 }
 
-// Prefill sizes (STORE, RESID_FIX, SWIGLU_Q8, QKV with at least one 128 x 64 tile per CU): the LDS-tiled
-// kernel, workgroups of 128 rows x 64 tokens (2 x 2 waves of 64 x 32; 165 VGPRs: three per CU). One K slice: each output
-// has exactly one writer, so RESID_FIX is a plain read-add-write. Measured at P = 2048: gate_up 247.6 us with
-// 128-token workgroups (two per CU) against 223.5 us with 64-token ones.
-template <int EPI>
-static int launch_mmq_big(GemvArgs a, hipStream_t s) {
-  const int rt = a.N / 128, tt2 = (a.T + 63) / 64;
-  if (rt * tt2 >= 768) {                           // three or more 64-token workgroups per CU
-    constexpr size_t lds2 = 2 * LdsTile<2, 2, 2, TILE_CB>::BUF;
-    hipLaunchKernelGGL((k_mmq_tile<2, 2, 2, EPI>), dim3(rt, 1, tt2), dim3(256), lds2, s, a);
-  } else {
-    // 32-token workgroups: twice the workgroups for grids that give CUs fewer than three 64-token ones, or
-    // an uneven number (N = 1536: 384 of them): measured at P = 2048, down 166.6 -> 150.6 us, qkv (512 ->
-    // 1024 workgroups) 49.9 -> 42.5 us; 64-row workgroups of 2 waves instead: down 186 us
-    constexpr size_t lds1 = 2 * LdsTile<2, 2, 1, TILE_CB>::BUF;
-    hipLaunchKernelGGL((k_mmq_tile<2, 2, 1, EPI>), dim3(rt, 1, (a.T + 31) / 32), dim3(256), lds1, s, a);
-  }
+// compute units of the current device, cached per device
+static int device_cus() {
+  static int cus[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!cus[dev] && hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus[dev] = 256;
+  return cus[dev];
+}
+
+template <int RT, int TN, int RW, int CW, int KW, int EPI>
+static int launch_mmq_t32(const GemvArgs& a, hipStream_t s) {
+  using L = T32<RT, TN, RW, CW, KW>;
+  hipLaunchKernelGGL((k_mmq_t32<RT, TN, RW, CW, KW, EPI>), dim3(a.N / L::ROWS, 1, (a.T + L::TOKS - 1) / L::TOKS),
+                     dim3(L::NTH), L::LDS, s, a);
   return launched("mmq");
+}
+
+// Up to 4096 rows (the qkv, o and down products) the tiles are few, so each wave takes one 32 x 32 tile.
+// From 512 tokens a wave takes the whole K, whatever T is, so that a prompt prefilled in chunks of 512 tokens and more
+// gives the sums of one chunk. us at 512 / 1024 / 2048 tokens, 1536 x 8960: 59 / 76 / 102 (16x16x32 tiles 89 / 110 /
+// 135; 128 x 64 workgroups of 32 x 64 tiles 90 / 91 / 121); 1536 x 1536: 14.6 / 19.3 / 24.7; 2048 x 1536: 12.9 / 16.9 / 27.8.
+// 256 to 511 tokens: four K waves per tile (333 tokens: 1536 x 8960 45 us against 59 with one and 89 for k_mmq<4>,
+// whose sums these are; 1536 x 1536 11.8 against 14.3 and 19.8).
+template <int EPI>
+static int launch_mmq_narrow(const GemvArgs& a, hipStream_t s) {
+  if (a.T >= 256 && a.T < 512) return launch_mmq_t32<1, 1, 1, 1, 4, EPI>(a, s);
+  if (a.N % 128) return launch_mmq_t32<1, 1, 2, 2, 1, EPI>(a, s);
+  return launch_mmq_t32<1, 1, 4, 1, 1, EPI>(a, s);
+}
+
+// Prefill sizes (STORE, RESID_FIX, SWIGLU_Q8, QKV): k_mmq_t32. Wide matrices take one wave per tile, so the summation
+// order is the same whatever the workgroup: 256 x 32, 128 x 64 or 128 x 128, by what the fullest CU costs (us for c
+// workgroups on it, from 17920 x 1536: 256 x 32 20 + 8 (c - 1), 128 x 64 18 + 7.2 (c - 1), 128 x 128 28 + 11 (c - 1)).
+// 17920 x 1536 (us; 16x16x32 tiles before): 77 tokens 20.3 (23.5), 200: 28 (34), 333: 39 (57), 2048: 160 (213).
+template <int EPI>
+static int launch_mmq_big(const GemvArgs& a, hipStream_t s) {
+  if constexpr (EPI != EPI_SWIGLU_Q8)
+    if (a.N <= 4096 || a.N % 128) return launch_mmq_narrow<EPI>(a, s);
+  const long cu = device_cus();
+  const auto full = [&](int rows, int toks) { return (double)(((long)a.N / rows * ((a.T + toks - 1) / toks) + cu - 1) / cu); };
+  const double c1 = 10.8 + 7.2 * full(128, 64), c2 = 17 + 11 * full(128, 128), c3 = 12 + 8 * full(256, 32);
+  if (a.N % 256 == 0 && c3 < c1 && c3 < c2) return launch_mmq_t32<2, 1, 4, 1, 1, EPI>(a, s);
+  if (c2 <= c1) return launch_mmq_t32<2, 2, 2, 2, 1, EPI>(a, s);
+  return launch_mmq_t32<2, 1, 2, 2, 1, EPI>(a, s);
 }
 
 // LOGITS over a large vocabulary (N % 128 == 0) for up to 64 tokens: the LDS-tiled kernel with all tokens
@@ -526,13 +553,13 @@ static int launch_mmq_logits_tile(const GemvArgs& a, hipStream_t s) {
   const dim3 grid(a.N / 128, 1, 1);
   if (a.T <= 16) {
     constexpr size_t lds = 2 * LdsTile<2, 1, 1, TILE_CB>::BUF;
-    hipLaunchKernelGGL((k_mmq_tile<2, 1, 1, EPI_LOGITS>), grid, dim3(128), lds, s, a);
+    hipLaunchKernelGGL((k_mmq_tile<2, 1, 1>), grid, dim3(128), lds, s, a);
   } else if (a.T <= 32) {
     constexpr size_t lds = 2 * LdsTile<2, 2, 1, TILE_CB>::BUF;
-    hipLaunchKernelGGL((k_mmq_tile<2, 2, 1, EPI_LOGITS>), grid, dim3(256), lds, s, a);
+    hipLaunchKernelGGL((k_mmq_tile<2, 2, 1>), grid, dim3(256), lds, s, a);
   } else {
     constexpr size_t lds = 2 * LdsTile<2, 2, 2, TILE_CB>::BUF;
-    hipLaunchKernelGGL((k_mmq_tile<2, 2, 2, EPI_LOGITS>), grid, dim3(256), lds, s, a);
+    hipLaunchKernelGGL((k_mmq_tile<2, 2, 2>), grid, dim3(256), lds, s, a);
   }
   return launched("mmq");
 }
@@ -600,14 +627,15 @@ static int launch_mmq_tg(const GemvArgs& a, int KS, hipStream_t s) {
   }
   if constexpr (EPI == EPI_LOGITS)
     if (a.N % 128 == 0 && a.N >= 128 * 256 && a.T <= 64) return launch_mmq_logits_tile(a, s);
-  // prefill sizes: the LDS-tiled kernel; from 512 tokens on always, so a prompt split into chunks of >= 512
-  // tokens computes every row with the same kernel (and the same summation order) as one chunk
+  // prefill sizes, and matrices with a 128 x 64 tile for every CU
   if constexpr (EPI == EPI_STORE || EPI == EPI_RESID_FIX || EPI == EPI_SWIGLU_Q8)
-    if (a.N % 128 == 0 && (a.T >= 512 || (a.N / 128) * ((a.T + 63) / 64) >= 256)) return launch_mmq_big<EPI>(a, s);
-  // up to 64 tokens (decode batches): 16-token workgroups, several per CU, hide each other's latencies;
-  // prefill sizes: 32- or 64-token workgroups reuse every staged weight block 2 or 4 times
+    if ((a.N % 128 == 0 && (a.N / 128) * ((a.T + 63) / 64) >= 256) || (a.T >= 256 && (EPI != EPI_SWIGLU_Q8 || a.N % 128 == 0)))
+      return launch_mmq_big<EPI>(a, s);
+  // up to 64 tokens (decode batches): 16-token workgroups, several per CU, hide each other's latencies; more: 32- or
+  // 64-token workgroups reuse every staged weight block 2 or 4 times
   if (a.T <= 64) return launch_mmq<1, EPI>(a, KS, s);
-  return a.T < 256 ? launch_mmq<2, EPI>(a, KS, s) : launch_mmq<4, EPI>(a, KS, s);
+  if constexpr (EPI == EPI_STORE || EPI == EPI_RESID_FIX) return launch_mmq<2, EPI>(a, KS, s);
+  else return a.T < 256 ? launch_mmq<2, EPI>(a, KS, s) : launch_mmq<4, EPI>(a, KS, s);
 }
 
 extern "C" int q355_mmq_q4_0_q8_1(const uint8_t* qs, const void* d, int N, int K, const int8_t* xq, const void* xds,
@@ -629,7 +657,7 @@ extern "C" int q355_mmq_q4_0_q8_1(const uint8_t* qs, const void* d, int N, int K
     case 6: {
       REQUIRE(yfix, "mmq_q4_0_q8_1: resid_fix needs yfix");
       a.yfix = (long long*)yfix;
-      int KS = T >= 256 ? 1 : 384 / groups;           // prefill sizes have parallelism enough
+      int KS = 384 / groups;                          // launch_mmq only: prefill sizes have parallelism enough
       KS = KS < 1 ? 1 : (KS > nb / 4 ? nb / 4 : KS);
       if (KS < 1) KS = 1;
       return launch_mmq_tg<EPI_RESID_FIX>(a, KS, s);
@@ -1025,16 +1053,6 @@ extern "C" int q355_mmq_qkv_rope(const uint8_t* qs, const void* d, int N, int K,
 extern "C" int64_t q355_attn_prefill_ws_bytes(int P, int max_ctx, int nh, int nkv) {
   if (P < 1 || max_ctx < P || nh < 1 || nkv < 1 || nh % nkv) return -1;
   return (int64_t)(pf_ws_floats((P + PF_QB - 1) / PF_QB, nkv, nh / nkv, pf_max_splits(0, max_ctx)) * sizeof(float));
-}
-
-// compute units of the current device (the persistent prefill attention's workgroups), cached per device
-static int device_cus() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cus[dev] && hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    cus[dev] = 256;
-  return cus[dev];
 }
 
 static int attn_prefill(const void* q, const void* kcache, const void* vcache, const int32_t* block_table, int pos0,

@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(NW * 64) k_mmq_reg(const GemvArgs a) {
   Q355_TRACE_POINT(5);
 }
 
-// Prefill-size GEMM tile: a workgroup computes (RW * 64 rows) x (CW * 16 TG tokens) with RW x CW = 4 waves,
+// LM head of a decode batch (up to 64 tokens): a workgroup computes (RW * 64 rows) x (CW * 16 TG tokens) with RW x CW waves,
 // each wave a 64 x 16 TG sub-tile (4 row tiles x TG token groups, 4 TG MFMAs per K block) over the full K slice.
 // K advances in chunks of CB blocks staged in LDS, double-buffered: the global loads of chunk c + 1 are
 // issued (16 B per lane, contiguous) before chunk c is computed, and written to the other buffer after.
@@ -571,9 +571,8 @@ __global__ void __launch_bounds__(NW * 64) k_mmq_reg(const GemvArgs a) {
 //   B  [CW*TG groups][CB][16 tokens][32 B] int8 activations; tokens 8..15 of a group swap their 16 B
 //                                          halves, so the two half-wave reads of a B operand use all banks
 //   X  [CB][CW*16*TG]                      activation scale / 16 (fp32)
-// Epilogues from registers: STORE, RESID_FIX (plain read-add-write: each output has one writer),
-// SWIGLU_Q8 (rows interleaved g0, u0, ...: each 64-row tile group is one Q8_1 block per token), LOGITS
-// (fp32 logits + one (max, row) partial per 64 rows and token, the layout of the other LOGITS kernels).
+// Epilogue from registers: fp32 logits and one (max, row) partial per 64 rows and token, the layout of the other LOGITS
+// kernels.
 template <int RW, int CW, int TG, int CB>
 struct LdsTile {
   static constexpr int TW = CW * 16 * TG;            // tokens per workgroup
@@ -582,7 +581,7 @@ struct LdsTile {
   static constexpr int BUF = A + W + B + X;
 };
 
-template <int RW, int CW, int TG, int EPI>
+template <int RW, int CW, int TG>
 __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
   constexpr int CB = TILE_CB;
   using L = LdsTile<RW, CW, TG, CB>;
@@ -709,118 +708,352 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
   for (int g = 0; g < TG; ++g) {
     const int tok = tok0 + wc * 16 * TG + g * 16 + li;
     const bool ok = tok < a.T;
-    if (EPI == EPI_STORE) {
-      if (ok)
+    // fp32 logits, and this wave's (max, lowest row) over its 64 rows: partial rt0 / 4 of N / 64
+    float bv = -INFINITY;
+    int bi = 0x7fffffff;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          *(float4*)(a.y + (size_t)tok * N + (rt0 + t) * 16 + 4 * lg) =
-              make_float4(acc[t][g][0], acc[t][g][1], acc[t][g][2], acc[t][g][3]);
-    } else if (EPI == EPI_RESID_FIX) {
-      if (ok) {
+    for (int t = 0; t < 4; ++t) {
+      if (ok && a.y)                                     // fp32 logits are optional: the argmax needs only partials
+        *(float4*)(a.y + (size_t)tok * N + (rt0 + t) * 16 + 4 * lg) =
+            make_float4(acc[t][g][0], acc[t][g][1], acc[t][g][2], acc[t][g][3]);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          long long* y = a.yfix + (size_t)tok * N + (rt0 + t) * 16 + 4 * lg;
-          if (gridDim.y == 1) {                      // this lane owns these 4 sums: plain read-add-write
-            longlong2* y2 = (longlong2*)y;
-            longlong2 p0 = y2[0], p1 = y2[1];
-            p0.x += to_fix((double)acc[t][g][0]); p0.y += to_fix((double)acc[t][g][1]);
-            p1.x += to_fix((double)acc[t][g][2]); p1.y += to_fix((double)acc[t][g][3]);
-            y2[0] = p0;
-            y2[1] = p1;
-          } else {
+      for (int v = 0; v < 4; ++v)                        // rows increase with (t, v): strict '>' keeps the lowest
+        if (acc[t][g][v] > bv) { bv = acc[t][g][v]; bi = (rt0 + t) * 16 + 4 * lg + v; }
+    }
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-              atomicAdd((unsigned long long*)(y + v), (unsigned long long)to_fix((double)acc[t][g][v]));
-          }
+    for (int o = 16; o <= 32; o <<= 1) {
+      const float ov = __shfl_xor(bv, o);
+      const int oi = __shfl_xor(bi, o);
+      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+    }
+    if (ok && lg == 0) {
+      const int np = N / 64;
+      a.pmax[(size_t)tok * np + rt0 / 4] = bv;
+      a.pidx[(size_t)tok * np + rt0 / 4] = bi;
+    }
+  }
+}
+
+// Prefill-size GEMM on v_mfma_i32_32x32x32_i8: a workgroup computes RW x CW wave tiles of (32 RT rows) x (32 TN
+// tokens) over the whole K. KW waves share a tile: each takes every KW-th K block, and their fp32 sums are added in f64
+// in the order of the waves. So a result depends on KW but not on the tile's or the workgroup's shape.
+// One 32-row tile of one Q4_0 block against 32 tokens is one MFMA. Lane l holds A[row l % 32][k = 16 (l / 32) .. +16]:
+// the low (lanes 0..31) or high nibbles of the row's 16 bytes as int8 16 (q - 8); B[k = 16 (l / 32) .. +16][token
+// l % 32]; and C[row 8 (v / 4) + 4 (l / 32) + v % 4][token l % 32], v = 0 .. 15. The d_w d_x of a tile come from one
+// fp16 product of depth 1 (v_mfma_f32_32x32x8_f16, the other k zero: exact in fp32, subnormal scales included).
+// acc += (d_w d_x) (16 dot') per block in fp32, in block order, and a final exact / 16: bit for bit the sums that the
+// 16x16x32 tile form gave.
+// What bounds it: VALU issue. A 32 x 32 tile and block needs 16 int32 -> fp32 converts and 16 fmas (each about 4.3
+// cycles of a SIMD while the matrix cores run), against 64 cycles of int8 and fp16 MFMAs that run beside them; the
+// unpacking, staging and epilogue add 15 more VALU instructions. fp32 scale products (v_mfma_f32_32x32x1) would hold
+// the VALU up: converts do not overlap with them. Counters at 17920 x 1536 x 2048 tokens: VALU 84 % busy.
+// Measured (us, 2048 tokens; before: 16x16x32 products with fp32 scale products): 17920 x 1536 213 -> 160 in 128 x 128
+// workgroups (174 in 128 x 64), 1536 x 8960 135 -> 102, 1536 x 1536 32 -> 25 and 2048 x 1536 34 -> 28 in 128 x 32 ones of
+// a 32 x 32 tile per wave.
+template <int RT, int TN, int RW, int CW, int KW>
+struct T32 {
+  static constexpr int CB = KW > 4 ? KW : 4;         // K blocks per LDS chunk
+  static constexpr int NTH = RW * CW * KW * 64, ROWS = RW * RT * 32, TOKS = CW * TN * 32;
+  static constexpr int BST = CB * 32 + 16;           // LDS bytes of one token's activations (padded: 16 rows cover all banks)
+  static constexpr int XST = TOKS + 16;              // LDS floats of one block's activation scales
+  static constexpr int A = ROWS * CB * 16, W = ROWS * CB * 4, B = TOKS * BST, X = CB * XST * 4;
+  static constexpr int BUF = A + W + B + X;
+  static constexpr int RED = KW > 1 ? KW * RW * CW * RT * TN * 16 * 64 * 4 : 0;       // sums exchanged at the end
+  static constexpr int LDS = 2 * BUF > RED ? 2 * BUF : RED;
+};
+
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v4h half0(unsigned bits) { return __builtin_bit_cast(v4h, make_uint2(bits, 0)); }
+
+// 16 bytes of nibbles -> this lane's 16 int8 values 16 (q - 8): sh = 4 for the low nibbles, 0 for the high ones
+__device__ __forceinline__ v4i snib16(uint4 w, int sh) {
+  const unsigned m = 0xF0F0F0F0u, f = 0x80808080u;
+  return (v4i){(int)(((w.x << sh) & m) ^ f), (int)(((w.y << sh) & m) ^ f), (int)(((w.z << sh) & m) ^ f),
+               (int)(((w.w << sh) & m) ^ f)};
+}
+
+template <int RT, int TN, int RW, int CW, int KW, int EPI>
+__global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a) {
+  using L = T32<RT, TN, RW, CW, KW>;
+  constexpr int CB = L::CB, NTH = L::NTH, ROWS = L::ROWS, TOKS = L::TOKS;
+  constexpr int PA = ROWS * CB, PW = ROWS * CB / 8, PB = TOKS * CB * 2, PX = TOKS * CB;   // staged pieces per chunk
+  static_assert((PA % NTH == 0 || PA <= NTH) && (PB % NTH == 0 || PB <= NTH) && PW <= NTH && (PX % NTH == 0 || PX <= NTH),
+                "staging shape");
+  constexpr int NA = PA > NTH ? PA / NTH : 1, NB = PB > NTH ? PB / NTH : 1, NX = PX > NTH ? PX / NTH : 1;
+  extern __shared__ __align__(16) char lds[];
+  const int K = a.K, nb = K / 32, N = a.N;
+  const KSlice ks(nb);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int lc = lane & 31, lh = lane >> 5;
+  const int wk = wv % KW, wr = wv / KW / CW, wc = wv / KW % CW;
+  const int tile0 = blockIdx.x * (ROWS / 16);         // first 16-row tile of the workgroup
+  const int tok0 = blockIdx.z * TOKS;
+
+  // Staging: every load is a workgroup-uniform base (advanced once per chunk) plus a 32-bit offset of this thread that
+  // stays the same for the whole K loop, so a chunk costs no address arithmetic. Tokens past T re-read the last one
+  // (never stored). A partial last chunk starts CB blocks before the slice's end and zeroes the scales of the blocks
+  // that are another chunk's or slice's (K < 32 CB: of the blocks past K, whose loads repeat the last one).
+  u32x4 rA[NA], rB[NB], rW = {};
+  unsigned rX[NX];
+  const int nt = min(TOKS, a.T - tok0);
+  unsigned oA[NA], oB[NB], oX[NX];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    const int p = min(tid + NTH * i, PA - 1);
+    oA[i] = (unsigned)((p / (CB * 16) * nb + min(p % (CB * 16) >> 4, nb - 1)) * 16 + (p & 15)) * 16;
+  }
+  const unsigned oW = (unsigned)((min(tid, PW - 1) / (CB * 2) * nb + min(tid % (CB * 2) >> 1, nb - 1)) * 2 + (tid & 1)) * 16;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int p = min(tid + NTH * i, PB - 1);
+    oB[i] = (unsigned)(min(p / (CB * 2), nt - 1) * K + min(p % (CB * 2) >> 1, nb - 1) * 32 + (p & 1) * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    const int p = min(tid + NTH * i, PX - 1);
+    oX[i] = (unsigned)(min(p / CB, nt - 1) * nb + min(p % CB, nb - 1)) * 4;
+  }
+#define Q355_T32_LOAD(c0)                                                                                       \
+  {                                                                                                             \
+    const int c_ = max(min((c0), ks.b1 - CB), 0), skip_ = (c0) - c_, end_ = ks.b1 - c_;                         \
+    const char* pA = (const char*)a.qs + ((size_t)tile0 * nb + c_) * 256;                                       \
+    const char* pW = (const char*)a.d + ((size_t)tile0 * nb + c_) * 32;                                         \
+    const char* pB = (const char*)a.xq + (size_t)tok0 * K + c_ * 32;                                            \
+    const char* pX = (const char*)a.xds + ((size_t)tok0 * nb + c_) * 4;                                         \
+    _Pragma("unroll") for (int i = 0; i < NA; ++i) rA[i] = *(const u32x4*)(pA + oA[i]);                   \
+    if (tid < PW) rW = *(const u32x4*)(pW + oW);                                                                \
+    _Pragma("unroll") for (int i = 0; i < NB; ++i) rB[i] = *(const u32x4*)(pB + oB[i]);                   \
+    _Pragma("unroll") for (int i = 0; i < NX; ++i) rX[i] = *(const unsigned*)(pX + oX[i]);                      \
+    if (skip_ || end_ < CB) {                         /* uniform: a partial last chunk */                       \
+      const int w_ = tid % (CB * 2) >> 1;                                                                       \
+      if (w_ < skip_ || w_ >= end_) rW = u32x4{};                                                               \
+      _Pragma("unroll") for (int i = 0; i < NX; ++i) {                                                          \
+        const int x_ = (tid + NTH * i) % CB;                                                                    \
+        if (x_ < skip_ || x_ >= end_) rX[i] = 0;                                                                \
+      }                                                                                                         \
+    }                                                                                                           \
+  }
+#define Q355_T32_STORE(base)                                                                                    \
+  {                                                                                                             \
+    char* b_ = (base);                                                                                          \
+    _Pragma("unroll") for (int i = 0; i < NA; ++i)                                                     \
+      if (PA % NTH == 0 || tid < PA) *(u32x4*)(b_ + (tid + NTH * i) * 16) = rA[i];                              \
+    if (tid < PW) {                                                                                             \
+      const int t = tid / (CB * 2), r = tid % (CB * 2);                                                         \
+      u32x4* dst = (u32x4*)(b_ + L::A + ((r >> 1) * ROWS + t * 16 + (r & 1) * 8) * 4);                          \
+      dst[0] = u32x4{rW.x & 0xFFFF, rW.x >> 16, rW.y & 0xFFFF, rW.y >> 16};                                \
+      dst[1] = u32x4{rW.z & 0xFFFF, rW.z >> 16, rW.w & 0xFFFF, rW.w >> 16};                                \
+    }                                                                                                           \
+    _Pragma("unroll") for (int i = 0; i < NB; ++i) {                                                      \
+      const int p = tid + NTH * i, j = p / (CB * 2), r = p % (CB * 2);                                          \
+      if (PB % NTH == 0 || tid < PB) *(u32x4*)(b_ + L::A + L::W + j * L::BST + r * 16) = rB[i];                                                \
+    }                                                                                                           \
+    _Pragma("unroll") for (int i = 0; i < NX; ++i) {                                                            \
+      const int p = tid + NTH * i;                                                                              \
+      if (PX % NTH == 0 || p < PX)                                                                              \
+        ((unsigned*)(b_ + L::A + L::W + L::B))[(p % CB) * L::XST + p / CB] = rX[i] & 0xFFFF;                    \
+    }                                                                                                           \
+  }
+
+  float acc[RT][TN][16];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int g = 0; g < TN; ++g)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[t][g][v] = 0.f;
+
+  if (ks.b0 < ks.b1) {
+    Q355_T32_LOAD(ks.b0);
+    Q355_T32_STORE(lds);
+  }
+  __syncthreads();
+  const int sh = lh ? 0 : 4;
+  const unsigned lo = lh ? 0u : ~0u;                  // scales enter as k = 0 of the fp16 product: lanes 0..31
+  int buf = 0;
+  for (int c0 = ks.b0; c0 < ks.b1; c0 += CB) {
+    const bool more = c0 + CB < ks.b1;                // uniform
+    if (more) Q355_T32_LOAD(c0 + CB);
+    const char* base = lds + buf * L::BUF;
+    const char* sA = base + (wr * RT * 2 + (lc >> 4)) * (CB * 256) + (lc & 15) * 16;
+    const unsigned* sW = (const unsigned*)(base + L::A) + wr * RT * 32 + lc;
+    const char* sB = base + L::A + L::W + (wc * TN * 32 + lc) * L::BST + lh * 16;
+    const unsigned* sX = (const unsigned*)(base + L::A + L::W + L::B) + wc * TN * 32 + lc;
+    const v16i zi = {};
+    const v16f zf = {};
+#pragma unroll RT* TN == 1 ? 2 : 1                     // one tile per wave: two blocks' operands and products in flight
+    for (int b = wk; b < CB; b += KW) {
+      v4i w[RT];
+      v4h dw[RT];
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        w[t] = snib16(*(const uint4*)(sA + t * 2 * (CB * 256) + b * 256), sh);
+        dw[t] = half0(sW[b * ROWS + t * 32] & lo);
+      }
+#pragma unroll
+      for (int g = 0; g < TN; ++g) {
+        const v4i x = *(const v4i*)(sB + g * 32 * L::BST + b * 32);
+        const v4h dx = half0(sX[b * L::XST + g * 32] & lo);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[t], x, zi, 0, 0, 0);
+          const v16f sc = __builtin_amdgcn_mfma_f32_32x32x8f16(dw[t], dx, zf, 0, 0, 0);
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[t][g][v] = fmaf(sc[v], (float)c[v], acc[t][g][v]);
         }
       }
-    } else if (EPI == EPI_LOGITS) {
-      // fp32 logits, and this wave's (max, lowest row) over its 64 rows: partial rt0 / 4 of N / 64
-      float bv = -INFINITY;
-      int bi = 0x7fffffff;
+    }
+    if (more) {
+      Q355_T32_STORE(lds + (buf ^ 1) * L::BUF);
+      __syncthreads();
+      buf ^= 1;
+    }
+  }
+#undef Q355_T32_LOAD
+#undef Q355_T32_STORE
+
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        if (ok && a.y)                                   // fp32 logits are optional: the argmax needs only partials
-          *(float4*)(a.y + (size_t)tok * N + (rt0 + t) * 16 + 4 * lg) =
-              make_float4(acc[t][g][0], acc[t][g][1], acc[t][g][2], acc[t][g][3]);
+  for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)                      // rows increase with (t, v): strict '>' keeps the lowest
-          if (acc[t][g][v] > bv) { bv = acc[t][g][v]; bi = (rt0 + t) * 16 + 4 * lg + v; }
+    for (int g = 0; g < TN; ++g)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[t][g][v] *= 0.0625f;
+
+  // A wave's epilogue takes groups of 4 rows x 32 tokens x 2 lane halves: group q = (token tile, row tile, u) holds rows
+  // 8 u + 4 lh .. + 3 of its tile. One K wave: its own RT * TN * 4 groups, from registers. More: all of them leave
+  // their sums in LDS and each adds up its share of the groups in the order of the waves.
+  constexpr int NG = RT * TN * 4 / KW;
+  static_assert(RT * TN * 4 % KW == 0, "whole groups per K wave");
+  typename std::conditional<KW == 1, float, double>::type sum[NG][4];
+  if constexpr (KW > 1) {
+    __syncthreads();
+    float4* red = (float4*)lds + (size_t)(wr * CW + wc) * (KW * RT * TN * 4 * 64) + lane;
+#pragma unroll
+    for (int g = 0; g < TN; ++g)
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          red[(wk * (RT * TN * 4) + (g * RT + t) * 4 + u) * 64] =
+              make_float4(acc[t][g][4 * u], acc[t][g][4 * u + 1], acc[t][g][4 * u + 2], acc[t][g][4 * u + 3]);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      for (int e = 0; e < 4; ++e) sum[i][e] = 0;
+#pragma unroll
+      for (int k = 0; k < KW; ++k) {
+        const float4 o = red[(k * (RT * TN * 4) + wk * NG + i) * 64];
+        sum[i][0] += o.x; sum[i][1] += o.y; sum[i][2] += o.z; sum[i][3] += o.w;
       }
+    }
+  } else {
 #pragma unroll
-      for (int o = 16; o <= 32; o <<= 1) {
-        const float ov = __shfl_xor(bv, o);
-        const int oi = __shfl_xor(bi, o);
-        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-      }
-      if (ok && lg == 0) {
-        const int np = N / 64;
-        a.pmax[(size_t)tok * np + rt0 / 4] = bv;
-        a.pidx[(size_t)tok * np + rt0 / 4] = bi;
-      }
-    } else if (EPI == EPI_QKV) {
-      // + bias, RoPE, fp16 q / K / V (one f64 -> fp16 rounding each, as k_qkv_finish): this lane's rows
-      // 4 lg + v of each tile are the RoPE pairs (v = 0, 1) and (2, 3) of the device row order
-      if (ok) {
-        const int nq = a.nh * HD, nk = a.nkv * HD;
-        const int pos = a.pos[tok];
-        const int pg = a.block_table[(size_t)(tok * a.seq_stride) * a.bt_stride + pos / PAGE];
+    for (int g = 0; g < TN; ++g)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < RT; ++t)
 #pragma unroll
-          for (int pp = 0; pp < 2; ++pp) {
-            const int row = (rt0 + t) * 16 + 4 * lg + 2 * pp;
-            const double v0 = (double)acc[t][g][2 * pp] + (double)a.aux[row];
-            const double v1 = (double)acc[t][g][2 * pp + 1] + (double)a.aux[row + 1];
-            if (row < nq + nk) {
-              const int i = (row % HD) >> 1;           // pair (dim i, dim i + 64)
-              const double c = a.rope_cos[(size_t)pos * (HD / 2) + i], sn = a.rope_sin[(size_t)pos * (HD / 2) + i];
-              const __half lo = half_rn(v0 * c - v1 * sn), hi = half_rn(v1 * c + v0 * sn);
-              __half* dst = row < nq ? a.qout + (size_t)tok * nq + (row / HD) * HD
-                                     : a.kcache + (((size_t)pg * a.nkv + (row - nq) / HD) * PAGE + pos % PAGE) * HD;
-              dst[i] = lo;
-              dst[i + HD / 2] = hi;
-              if (row < nq && a.qout64) {
-                double* d64 = a.qout64 + (size_t)tok * nq + (row / HD) * HD;
-                d64[i] = (double)__half2float(lo);
-                d64[i + HD / 2] = (double)__half2float(hi);
-              }
-            } else {
-              const int rv = row - nq - nk;
-              __half2* vd = (__half2*)(a.vcache + (((size_t)pg * a.nkv + rv / HD) * PAGE + pos % PAGE) * HD + rv % HD);
-              *vd = __halves2half2(half_rn(v0), half_rn(v1));
-            }
-          }
-      }
-    } else if (EPI == EPI_SWIGLU_Q8) {
-      // this lane holds outputs 8t + 2lg, 8t + 2lg + 1 of its wave's 32; the 4 lanes of token li hold all 32
-      float o[4][2];
-      float amax = 0.f;
+        for (int v = 0; v < 16; ++v) sum[(g * RT + t) * 4 + v / 4][v % 4] = acc[t][g][v];
+  }
+  const int rowb = tile0 * 16 + wr * RT * 32 + 4 * lh, tokb = tok0 + wc * TN * 32 + lc;
+  if constexpr (EPI == EPI_SWIGLU_Q8) {
+    // the wave's 64 rows are one Q8_1 block of 32 outputs per token; lanes l and l ^ 32 hold 16 each: outputs
+    // 16 t + 4 u + 2 lh, + 1 in rows 8 u + 4 lh .. of tile t
+    static_assert(EPI != EPI_SWIGLU_Q8 || (RT == 2 && KW == 1), "64 rows per wave");
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        o[t][0] = silu_mul_f(acc[t][g][0], acc[t][g][1]);
-        o[t][1] = silu_mul_f(acc[t][g][2], acc[t][g][3]);
-        amax = fmaxf(amax, fmaxf(fabsf(o[t][0]), fabsf(o[t][1])));
-      }
-      amax = fmaxf(amax, __shfl_xor(amax, 16));
-      amax = fmaxf(amax, __shfl_xor(amax, 32));
+    for (int g = 0; g < TN; ++g) {
+      const int tok = tokb + 32 * g;
+      float o[2][4][2], amax = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const auto& s = sum[(g * 2 + t) * 4 + u];
+          o[t][u][0] = silu_mul_f(s[0], s[1]);
+          o[t][u][1] = silu_mul_f(s[2], s[3]);
+          amax = fmaxf(amax, fmaxf(fabsf(o[t][u][0]), fabsf(o[t][u][1])));
+        }
+      auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
+      amax = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
       const float d32 = q8_scale(amax);
       int sq = 0;
-      unsigned short pk[4];
+      unsigned pk[2][4], word[4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int q0 = q8_code(o[t][0], d32), q1 = q8_code(o[t][1], d32);
-        sq += q0 + q1;
-        pk[t] = (unsigned short)((q0 & 255) | ((q1 & 255) << 8));
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int q0 = q8_code(o[t][u][0], d32), q1 = q8_code(o[t][u][1], d32);
+          sq += q0 + q1;
+          pk[t][u] = (q0 & 255) | ((q1 & 255) << 8);
+        }
+      // lanes 0..31 collect tile 0's 16 codes, lanes 32..63 tile 1's: one 16-byte store each
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const auto s = __builtin_amdgcn_permlane32_swap(pk[0][u], pk[1][u], false, false);
+        word[u] = s[0] | (s[1] << 16);
       }
-      sq += __shfl_xor(sq, 16);
-      sq += __shfl_xor(sq, 32);
-      if (ok) {
-        const int Nout = N / 2, ob = rt0 / 4;        // output Q8_1 block of this wave's 64 rows
-        int8_t* dst = a.oq + (size_t)tok * Nout + ob * 32 + 2 * lg;
+      r = __builtin_amdgcn_permlane32_swap((unsigned)sq, (unsigned)sq, false, false);
+      sq = (int)r[0] + (int)r[1];
+      if (tok < a.T) {
+        const int Nout = N / 2, ob = tile0 / 4 + wr;   // output Q8_1 block of this wave's 64 rows
+        *(uint4*)(a.oq + (size_t)tok * Nout + ob * 32 + 16 * lh) = make_uint4(word[0], word[1], word[2], word[3]);
+        if (!lh) a.ods[(size_t)tok * (Nout / 32) + ob] = __halves2half2(__float2half_rn(d32), q8_s16(d32, sq));
+      }
+    }
+    return;
+  }
+  int tokp = -1, pos = 0, pg = 0;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) *(unsigned short*)(dst + 8 * t) = pk[t];
-        if (lg == 0) a.ods[(size_t)tok * (Nout / 32) + ob] = __halves2half2(__float2half_rn(d32), q8_s16(d32, sq));
+  for (int i = 0; i < NG; ++i) {
+    const int q = wk * NG + i, tok = tokb + 32 * (q / (4 * RT)), row = rowb + 32 * (q / 4 % RT) + 8 * (q & 3);
+    if (tok >= a.T) continue;
+    const auto& s = sum[i];
+    if constexpr (EPI == EPI_STORE) {
+      *(float4*)(a.y + (size_t)tok * N + row) = make_float4(s[0], s[1], s[2], s[3]);
+    } else if constexpr (EPI == EPI_RESID_FIX) {         // this lane owns these 4 sums: plain read-add-write
+      longlong2* y2 = (longlong2*)(a.yfix + (size_t)tok * N + row);
+      longlong2 p0 = y2[0], p1 = y2[1];
+      p0.x += to_fix((double)s[0]); p0.y += to_fix((double)s[1]);
+      p1.x += to_fix((double)s[2]); p1.y += to_fix((double)s[3]);
+      y2[0] = p0;
+      y2[1] = p1;
+    } else if constexpr (EPI == EPI_QKV) {
+      // + bias, RoPE, fp16 q / K / V (one f64 -> fp16 rounding each, as k_qkv_finish): the lane's 4 rows are two RoPE
+      // pairs of the device row order
+      const int nq = a.nh * HD, nk = a.nkv * HD;
+      if (tok != tokp) {
+        tokp = tok;
+        pos = a.pos[tok];
+        pg = a.block_table[(size_t)(tok * a.seq_stride) * a.bt_stride + pos / PAGE];
+      }
+      const float* bias = a.aux + row;
+      const double v[4] = {(double)s[0] + (double)bias[0], (double)s[1] + (double)bias[1], (double)s[2] + (double)bias[2],
+                           (double)s[3] + (double)bias[3]};
+      if (row < nq + nk) {
+        const int i0 = (row % HD) >> 1;                  // pairs (dim i0, i0 + 64) and (i0 + 1, i0 + 65)
+        const float* rc = a.rope_cos + (size_t)pos * (HD / 2) + i0;
+        const float* rs = a.rope_sin + (size_t)pos * (HD / 2) + i0;
+        const double c0 = rc[0], c1 = rc[1], s0 = rs[0], s1 = rs[1];
+        const __half2 lo = __halves2half2(half_rn(v[0] * c0 - v[1] * s0), half_rn(v[2] * c1 - v[3] * s1));
+        const __half2 hi = __halves2half2(half_rn(v[1] * c0 + v[0] * s0), half_rn(v[3] * c1 + v[2] * s1));
+        __half* dst = row < nq ? a.qout + (size_t)tok * nq + (row / HD) * HD
+                               : a.kcache + (((size_t)pg * a.nkv + (row - nq) / HD) * PAGE + pos % PAGE) * HD;
+        *(__half2*)(dst + i0) = lo;
+        *(__half2*)(dst + i0 + HD / 2) = hi;
+        if (row < nq && a.qout64) {
+          double* d64 = a.qout64 + (size_t)tok * nq + (row / HD) * HD + i0;
+          d64[0] = (double)__low2float(lo);
+          d64[1] = (double)__high2float(lo);
+          d64[HD / 2] = (double)__low2float(hi);
+          d64[HD / 2 + 1] = (double)__high2float(hi);
+        }
+      } else {
+        const int rv = row - nq - nk;
+        __half2* vd = (__half2*)(a.vcache + (((size_t)pg * a.nkv + rv / HD) * PAGE + pos % PAGE) * HD + rv % HD);
+        vd[0] = __halves2half2(half_rn(v[0]), half_rn(v[1]));
+        vd[1] = __halves2half2(half_rn(v[2]), half_rn(v[3]));
       }
     }
   }

@@ -301,11 +301,13 @@ def flash_prefill_v3_source(maxlen: int = 4096, q8: bool = True) -> KernelSpec:
     return KernelSpec("q355_attn_prefill_q8_1" if q8 else "q355_attn_prefill")
 
 
-# chunks of at least this many tokens run the QKV product on the LDS-tiled kernel with the finish in its
-# epilogue (q355_mmq_qkv_rope); shorter ones keep the K-split product into the int64 accumulator plus
-# q355_qkv_finish, which has parallelism enough at small P. From 512 tokens on every product of a chunk runs
-# the LDS-tiled kernel, so chunking a prompt into pieces of >= 512 tokens gives the same results bit for bit.
-QKV_FUSED_MIN_P = 512
+# chunks of at least this many tokens, and those of up to QKV_FUSED_SMALL_P, run the QKV product with the finish in its
+# epilogue (q355_mmq_qkv_rope: one launch, no int64 accumulator; 333 tokens: 12 us against 24 + 6). Those between keep
+# the K-split product into the int64 accumulator plus q355_qkv_finish, which accumulates in f64 (up to 64 tokens) or in
+# short fp32 chains. From 512 tokens on no product's summation order depends on the chunk, so chunking a prompt into
+# pieces of >= 512 tokens gives the same results bit for bit.
+QKV_FUSED_MIN_P = 256
+QKV_FUSED_SMALL_P = 32
 
 
 class Prefill:
@@ -313,7 +315,7 @@ class Prefill:
 
     chunk(ids, pos0) runs P prompt tokens at positions pos0 .. pos0 + P - 1 through all layers at once:
       embed -> per layer: rmsnorm_fix_q8_1, MMQ qkv with bias + RoPE + K/V write in its epilogue
-      (P >= QKV_FUSED_MIN_P; else MMQ qkv into an int64 accumulator + qkv_finish),
+      (P >= QKV_FUSED_MIN_P or P <= QKV_FUSED_SMALL_P; else MMQ qkv into an int64 accumulator + qkv_finish),
       attn_prefill_q8_1 (causal, fp16 MFMA, Q8_1 output), MMQ o (+= h), rmsnorm_fix_q8_1, MMQ gate_up (SwiGLU -> Q8_1),
       MMQ down (+= h) -> final norm + head on the last token -> dec.tok = argmax, dec.pos = pos0 + P.
     The decoder then continues greedy decode from that state."""
@@ -345,7 +347,7 @@ class Prefill:
         L = m.layers[i]
         call("q355_rmsnorm_fix_q8_1", ptr(self.h), ptr(L["ln1"]), ptr(self.xq), ptr(self.xds), P, c.H, c.eps)
         W = L["qkv"]
-        if P >= QKV_FUSED_MIN_P:
+        if P >= QKV_FUSED_MIN_P or P <= QKV_FUSED_SMALL_P:
             # one writer per output: the finish (bias, RoPE, K/V write) runs in the GEMM epilogue
             call("q355_mmq_qkv_rope", ptr(W.qs), ptr(W.d), W.N, W.K, ptr(self.xq), ptr(self.xds), P, ptr(L["qkv_b"]),
                  ptr(m.cos), ptr(m.sin), ptr(self.pos), ptr(d.block_table), d.max_chunks, 0, ptr(d.kc[i]),

@@ -1,0 +1,92 @@
+"""The prefill products on 32 x 32 x 32 int8 tiles (k_mmq_t32) at the sizes where they can go wrong: K shorter than a
+staged chunk of 4 blocks, K that ends inside one, token counts around a tile, every tile form, activations of -128
+and subnormal scales.
+
+Reference: the exact block dots with their scales, summed in float64. The kernel adds the nb exact terms of an output in
+fp32 (possibly as four chains, joined in f64), so |error| <= (nb + 1) 2^-24 sum |terms| to first order; 2^-23 covers the rest."""
+import numpy as np
+import pytest
+
+from lab import qwen_model as QM
+from lab.hip import call, ptr
+from oracle import quant as OQ
+
+pytestmark = pytest.mark.gpu
+
+
+def problem(N, K, T, seed):
+    rng = np.random.default_rng(seed)
+    nb = K // 32
+    qs = rng.integers(0, 256, (N, nb, 16), dtype=np.uint8)
+    dw = (rng.standard_normal((N, nb)) * 0.01).astype(np.float16)
+    dw[rng.random((N, nb)) < 0.1] = np.float16(3e-6)                    # subnormal in fp16
+    xq = rng.integers(-128, 128, (T, K), dtype=np.int8)
+    dx = (rng.random((T, nb)) * 0.02).astype(np.float16)
+    dx[rng.random((T, nb)) < 0.1] = np.float16(1e-5)
+    wb = np.concatenate([dw.view(np.uint8).reshape(N, nb, 2), qs], axis=2).reshape(-1, 18)
+    return wb, dw, xq, dx
+
+
+def reference(wb, dw, xq, dx, N, K, T):
+    nb = K // 32
+    qw = OQ.q4_0_blocks(wb)[1].reshape(N, K)
+    sq = xq.reshape(T, nb, 32).astype(np.int64).sum(axis=2)
+    y, mag = np.zeros((T, N)), np.zeros((T, N))
+    for b in range(nb):
+        dot = OQ.block_dots(qw[:, 32 * b:32 * b + 32], xq[:, 32 * b:32 * b + 32])[:, :, 0] - 8 * sq[:, b:b + 1]
+        term = dot * dw[:, b].astype(np.float64)[None] * dx[:, b].astype(np.float64)[:, None]
+        y += term
+        mag += np.abs(term)
+    return y, (nb + 1) * 2.0 ** -23 * mag
+
+
+# dispatch: up to 4096 rows one 32 x 32 tile per wave, with four K waves from 256 to 511 tokens (128- or, for an odd
+# multiple of 64 rows, 64-row workgroups from 512); wider 256 x 32, 128 x 64 or 128 x 128 workgroups
+@pytest.mark.parametrize("N,K,T", [(64, 32, 256), (128, 288, 257), (1536, 160, 333), (192, 96, 511), (4096, 64, 300),
+                                   (128, 32, 512), (64, 96, 545), (192, 128, 513), (128, 160, 575),
+                                   (128, 288, 576), (4096, 96, 513), (2048, 32, 1100),
+                                   (4224, 32, 512), (4224, 160, 513), (4224, 416, 640), (4160, 96, 300),
+                                   (17920, 96, 65), (17920, 32, 333)])
+def test_mmq_t32_store_and_resid(cuda, N, K, T):
+    import torch
+    wb, dw, xq, dx = problem(N, K, T, N + K + T)
+    W = QM.Q4Mat(wb, N, K, "cuda")
+    xq_d = torch.from_numpy(xq).cuda()
+    xds_d = torch.from_numpy(np.stack([dx, np.zeros_like(dx)], -1)).cuda()
+    ref, bound = reference(wb, dw, xq, dx, N, K, T)
+    y = torch.full((T, N), float("nan"), device=cuda)
+    call("q355_mmq_q4_0_q8_1", ptr(W.qs), ptr(W.d), N, K, ptr(xq_d), ptr(xds_d), T, 0, ptr(y), None, None, None, None, None)
+    h0 = torch.from_numpy(np.random.default_rng(T).integers(-2 ** 40, 2 ** 40, (T, N))).cuda()
+    h = h0.clone()
+    call("q355_mmq_q4_0_q8_1", ptr(W.qs), ptr(W.d), N, K, ptr(xq_d), ptr(xds_d), T, 6, None, ptr(h), None, None, None, None)
+    torch.cuda.synchronize()
+    assert (np.abs(y.cpu().numpy() - ref) <= bound).all()
+    got = (h - h0).cpu().numpy() / QM.FIX_SCALE                          # 2^-49: the fixed-point rounding
+    assert (np.abs(got - ref) <= bound + 2.0 ** -48).all()
+
+
+@pytest.mark.parametrize("T", [512, 577, 1100])
+def test_mmq_t32_swiglu_is_the_quantized_store(cuda, T):
+    """SWIGLU_Q8 gives the Q8_1 rule of silu(g) u: codes within one step of those of the STORE sums, and d equal to the
+    fp16 of their block maximum / 127 within the error of the hardware exp2 and reciprocal (about 2e-6 relative)."""
+    import torch
+    N, K = 4224, 160
+    wb, dw, xq, dx = problem(N, K, T, T)
+    W = QM.Q4Mat(wb, N, K, "cuda")
+    xq_d = torch.from_numpy(xq).cuda()
+    xds_d = torch.from_numpy(np.stack([dx, np.zeros_like(dx)], -1)).cuda()
+    y = torch.zeros(T, N, device=cuda)
+    oq = torch.zeros(T, N // 2, dtype=torch.int8, device=cuda)
+    ods = torch.zeros(T, N // 64, 2, dtype=torch.float16, device=cuda)
+    args = ptr(W.qs), ptr(W.d), N, K, ptr(xq_d), ptr(xds_d), T
+    call("q355_mmq_q4_0_q8_1", *args, 0, ptr(y), None, None, None, None, None)
+    call("q355_mmq_q4_0_q8_1", *args, 7, None, None, ptr(oq), ptr(ods), None, None)
+    torch.cuda.synchronize()
+    g, u = y.double()[:, 0::2], y.double()[:, 1::2]
+    m = (g / (1 + torch.exp(-g)) * u).cpu().numpy()
+    q, d, s = OQ.quantize_q8_1(m.astype(np.float32))
+    dq = np.abs(oq.cpu().numpy().astype(int) - q)
+    assert dq.max() <= 1 and (dq > 0).mean() < 1e-3
+    ds = ods.cpu().numpy().astype(np.float64)
+    assert (np.abs(ds[..., 0] - d) <= 2.0 ** -10 * np.abs(d) + 2.0 ** -24).all()
+    assert np.allclose(ds[..., 1], ds[..., 0] * oq.cpu().numpy().reshape(T, -1, 32).sum(2), rtol=2e-3, atol=1e-3)
