@@ -848,12 +848,18 @@ extern "C" int q355_mmq_q6k_logits(const uint8_t* lo, const uint8_t* hi, const i
   GemvArgs a = {};
   a.qs = lo; a.qhi = hi; a.qsc = (const uint8_t*)sc; a.d = (const __half*)d; a.N = V; a.K = K; a.T = T;
   a.xq = xq; a.xds = (const half2*)xds; a.y = y; a.pmax = pmax; a.pidx = pidx;
-  const int TT = T <= 16 ? 16 : 32;
-  const size_t lds = (size_t)TT * (K + Q6M_XPAD) + (size_t)TT * (K / 32) * sizeof(float);
-  if (T <= 16)
-    hipLaunchKernelGGL(k_mmq_q6k_logits<1>, dim3(V / 64), dim3(Q6M_WAVES * 64), lds, (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(k_mmq_q6k_logits<2>, dim3(V / 64), dim3(Q6M_WAVES * 64), lds, (hipStream_t)stream, a);
+  // 8 waves share a staging of the activations where the vocabulary allows
+  const int TT = T <= 8 ? 8 : T <= 16 ? 16 : 32;
+  const size_t lds = (size_t)TT * (K + q6m_pad(T <= 8)) + (size_t)TT * (K / 32) * sizeof(float);
+  const auto go = [&](auto nw) {
+    constexpr int NW = decltype(nw)::value;
+    const dim3 grid(V / (16 * NW)), block(NW * 64);
+    if (T <= 8) hipLaunchKernelGGL((k_mmq_q6k_logits<0, NW>), grid, block, lds, (hipStream_t)stream, a);
+    else if (T <= 16) hipLaunchKernelGGL((k_mmq_q6k_logits<1, NW>), grid, block, lds, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL((k_mmq_q6k_logits<2, NW>), grid, block, lds, (hipStream_t)stream, a);
+  };
+  if (V % 128 == 0) go(std::integral_constant<int, 8>());
+  else go(std::integral_constant<int, 4>());
   return launched("mmq_q6k_logits");
 }
 

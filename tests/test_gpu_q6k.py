@@ -92,6 +92,37 @@ def test_mmq_q6k_logits(cuda, N, K, T):
     assert np.array_equal(pidx.cpu().numpy(), parts.argmax(axis=2) + 64 * np.arange(N // 64)[None])
 
 
+@pytest.mark.parametrize("N", [64, 192, 256])
+@pytest.mark.parametrize("K,T", [(256, 1), (512, 8), (256, 9), (768, 16), (1536, 17), (1280, 32)])
+def test_mmq_q6k_logits_forms(cuda, N, K, T):
+    """Every form of the batched Q6_K head (up to 8, 16 and 32 tokens; 4- and 8-wave workgroups; 2 to 12 groups of four
+    blocks) on extreme operands: activations down to -128, scales -128 and 127, all v. Each output is a sum of K / 32
+    exact terms in fp32 chains: |error| <= (K / 32 + 3) 2^-24 sum |terms| to first order; 2^-23 covers the rest."""
+    import torch
+    rng = np.random.default_rng(N + K + T)
+    b = random_q6_k(N * K // 256, rng, d=0.0005)
+    b[::7, 192:208] = np.array([128, 127] * 8, np.uint8)               # sub-block scales -128, 127
+    W = QM.Q6KMat(b, N, K, "cuda")
+    q = rng.integers(-128, 128, (T, K)).astype(np.int8)
+    d = (rng.random((T, K // 32)) * 0.02).astype(np.float16)
+    xq = torch.from_numpy(q).cuda()
+    xds = torch.from_numpy(np.stack([d, np.zeros_like(d)], -1)).cuda()
+    y = torch.full((T, N), float("nan"), device=cuda)
+    pmax = torch.zeros(T, N // 64, device=cuda)
+    pidx = torch.zeros(T, N // 64, dtype=torch.int32, device=cuda)
+    call("q355_mmq_q6k_logits", ptr(W.lo), ptr(W.hi), ptr(W.sc), ptr(W.d), N, K, ptr(xq), ptr(xds), T, ptr(y),
+         ptr(pmax), ptr(pidx))
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    w = OQ.dequant_q6_k(b, (N, K)).astype(np.float64).reshape(N, K // 32, 32)
+    x = q.astype(np.float64).reshape(T, K // 32, 32) * d.astype(np.float64)[..., None]
+    terms = np.einsum("nbi,tbi->tnb", w, x)
+    assert (np.abs(got - terms.sum(2)) <= (K // 32 + 3) * 2.0 ** -23 * np.abs(terms).sum(2)).all()
+    parts = got.reshape(T, N // 64, 64)
+    assert np.array_equal(pmax.cpu().numpy(), parts.max(axis=2))
+    assert np.array_equal(pidx.cpu().numpy(), parts.argmax(axis=2) + 64 * np.arange(N // 64)[None])
+
+
 @pytest.mark.parametrize("B", [8, 32])
 def test_batched_decode_with_q6k_head(cuda, B):
     """BatchedDecoder with llama.cpp's Q6_K output.weight (int8 MMQ layers, Q6_K MFMA head), teacher-forced
