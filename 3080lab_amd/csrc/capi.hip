@@ -631,10 +631,22 @@ static int launch_mmq_tg(const GemvArgs& a, int KS, hipStream_t s) {
   if constexpr (EPI == EPI_STORE || EPI == EPI_RESID_FIX || EPI == EPI_SWIGLU_Q8)
     if ((a.N % 128 == 0 && (a.N / 128) * ((a.T + 63) / 64) >= 256) || (a.T >= 256 && (EPI != EPI_SWIGLU_Q8 || a.N % 128 == 0)))
       return launch_mmq_big<EPI>(a, s);
-  // up to 64 tokens (decode batches): 16-token workgroups, several per CU, hide each other's latencies; more: 32- or
-  // 64-token workgroups reuse every staged weight block 2 or 4 times
+  // up to 64 tokens (decode batches): 16-token workgroups, several per CU, hide each other's latencies; what is left of
+  // the larger calls: 32- or 64-token workgroups reuse every staged weight block 2 or 4 times
   if (a.T <= 64) return launch_mmq<1, EPI>(a, KS, s);
-  if constexpr (EPI == EPI_STORE || EPI == EPI_RESID_FIX) return launch_mmq<2, EPI>(a, KS, s);
+  if constexpr (EPI == EPI_RESID_FIX) {                // 65 to 255 tokens
+    const int per = (a.K / 32 + KS - 1) / KS;
+    // longer slices (the down product) stay on the 16-token kernel: a wave would run its 18 blocks one latency after
+    // another (1536 x 8960, 77 / 200 tokens: 25.5 / 48 us against 23.5 / 41)
+    if (per > 4) return launch_mmq<2, EPI>(a, KS, s);
+    GemvArgs b = a;
+    b.mmq_chunk = per;
+    hipLaunchKernelGGL(k_mmq_s32, dim3(a.N / 32, 1, (a.T + 31) / 32), dim3(S32_KW * 64), 0, s, b);
+    return launched("mmq");
+  }
+  // STORE has no K split over the grid: 64 x 32 tiles of eight K waves, their fp32 chains added in f64 (us at 77 tokens,
+  // k_mmq<2> with four: 1536 x 8960 25 against 56, 1536 x 1536 7.7 against 12.3)
+  if constexpr (EPI == EPI_STORE) return launch_mmq_t32<2, 1, 1, 1, 8, EPI>(a, s);
   else return a.T < 256 ? launch_mmq<2, EPI>(a, KS, s) : launch_mmq<4, EPI>(a, KS, s);
 }
 

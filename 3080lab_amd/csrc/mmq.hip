@@ -1059,4 +1059,83 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
   }
 }
 
+// RESID_FIX for 65 to 255 tokens over a short K (the qkv and o products), where the tiles are few: the K slices of
+// k_mmq_reg's grid (a.mmq_chunk <= 4 blocks each; the fp32 block terms of a slice added in f64 and rounded to fixed point:
+// the same bytes), but a slice is one wave's 32 x 32 tile, and the workgroup's waves take the slices of one tile and add
+// them through LDS, so an output has one writer: the int64 atomics of the slices (one per output and slice) had been
+// most of the time. A wave loads the blocks of two slices before its first product: one memory latency.
+// Measured (us at 77 / 150 / 250 tokens; k_mmq_reg with atomics before): 1536 x 1536 9.6 / 9.9 / 17.2 (11.8 / 20 / 31), 2048 x
+// 1536 9.8 / 16.5 / 17.7 (16.5 / 24 / 38). Bounded by two memory latencies and the f64 rounding; past one workgroup per
+// CU (registers) by their rounds.
+constexpr int S32_KW = 6;
+
+__global__ void __launch_bounds__(S32_KW * 64) k_mmq_s32(const GemvArgs a) {
+  __shared__ unsigned long long part[16][64];
+  const int K = a.K, nb = K / 32, N = a.N, per = a.mmq_chunk;
+  const int tid = threadIdx.x, lane = tid & 63, wk = tid >> 6, lc = lane & 31, lh = lane >> 5;
+  const int tok0 = blockIdx.z * 32, row0 = blockIdx.x * 32;
+  const int tok = min(tok0 + lc, a.T - 1);              // tokens past T repeat the last one, never stored
+  const char* gA = (const char*)a.qs + ((size_t)(row0 / 16 + (lc >> 4)) * nb * 16 + (lc & 15)) * 16;
+  const char* gW = (const char*)a.d + ((size_t)(row0 / 16 + (lc >> 4)) * nb * 16 + (lc & 15)) * 2;
+  const char* gB = (const char*)a.xq + (size_t)tok * K + lh * 16;
+  const char* gX = (const char*)a.xds + (size_t)tok * nb * 4;
+  const int sh = lh ? 0 : 4;
+  const unsigned lo = lh ? 0u : 0xFFFFu;                // scales enter as k = 0 of the fp16 product: lanes 0..31
+  const v16i zi = {};
+  const v16f zf = {};
+  long long sum[16];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) sum[v] = 0;
+  for (int b0 = wk * per; b0 < nb; b0 += 2 * S32_KW * per) {          // two of this wave's slices at a time
+    u32x4 w[2][4];
+    v4i x[2][4];
+    unsigned dw[2][4], dx[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int b = min(b0 + i * S32_KW * per + min(e, per - 1), nb - 1);
+        w[i][e] = *(const u32x4*)(gA + (size_t)b * 256);
+        x[i][e] = *(const v4i*)(gB + (size_t)b * 32);
+        dw[i][e] = *(const unsigned short*)(gW + (size_t)b * 32);
+        dx[i][e] = *(const unsigned*)(gX + (size_t)b * 4);
+      }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int s0 = b0 + i * S32_KW * per, s1 = min(s0 + per, nb);
+      if (s0 >= nb) break;                                            // uniform
+      double s[16];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) s[v] = 0.0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (s0 + e < s1) {                                            // uniform
+          const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+              snib16(make_uint4(w[i][e].x, w[i][e].y, w[i][e].z, w[i][e].w), sh), x[i][e], zi, 0, 0, 0);
+          const v16f sc = __builtin_amdgcn_mfma_f32_32x32x8f16(half0(dw[i][e] & lo), half0(dx[i][e] & lo), zf, 0, 0, 0);
+#pragma unroll
+          for (int v = 0; v < 16; ++v) s[v] += (double)(sc[v] * 0.0625f * (float)c[v]);
+        }
+#pragma unroll
+      for (int v = 0; v < 16; ++v) sum[v] += to_fix(s[v]);
+    }
+  }
+  for (int e = tid; e < 16 * 64; e += S32_KW * 64) part[e >> 6][e & 63] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 16; ++v) atomicAdd(&part[v][lane], (unsigned long long)sum[v]);      // integers: any order
+  __syncthreads();
+  for (int e = tid; e < 512; e += S32_KW * 64) {                      // 2 consecutive rows of one token
+    const int r = (e & 15) * 2, t = e >> 4;
+    const int pv = 4 * (r >> 3) + (r & 3), pl = t + 32 * ((r >> 2) & 1);
+    if (tok0 + t < a.T) {
+      longlong2* y = (longlong2*)(a.yfix + (size_t)(tok0 + t) * N + row0 + r);
+      longlong2 h = *y;
+      h.x += (long long)part[pv][pl];
+      h.y += (long long)part[pv + 1][pl];
+      *y = h;
+    }
+  }
+}
+
 }  // namespace q355

@@ -40,9 +40,11 @@ def reference(wb, dw, xq, dx, N, K, T):
     return y, (nb + 1) * 2.0 ** -23 * mag
 
 
-# dispatch: up to 4096 rows one 32 x 32 tile per wave, with four K waves from 256 to 511 tokens (128- or, for an odd
-# multiple of 64 rows, 64-row workgroups from 512); wider 256 x 32, 128 x 64 or 128 x 128 workgroups
-@pytest.mark.parametrize("N,K,T", [(64, 32, 256), (128, 288, 257), (1536, 160, 333), (192, 96, 511), (4096, 64, 300),
+# dispatch: 65 to 255 tokens: RESID_FIX slices of one tile per workgroup (k_mmq_s32), STORE eight K waves; then up to 4096
+# rows one 32 x 32 tile per wave, with four K waves from 256 to 511 tokens (128- or, for an odd multiple of 64 rows, 64-row
+# workgroups from 512); wider 256 x 32, 128 x 64 or 128 x 128 workgroups
+@pytest.mark.parametrize("N,K,T", [(64, 32, 65), (128, 288, 97), (1536, 160, 200), (192, 8960, 70), (4096, 96, 255),
+                                   (64, 32, 256), (128, 288, 257), (1536, 160, 333), (192, 96, 511), (4096, 64, 300),
                                    (128, 32, 512), (64, 96, 545), (192, 128, 513), (128, 160, 575),
                                    (128, 288, 576), (4096, 96, 513), (2048, 32, 1100),
                                    (4224, 32, 512), (4224, 160, 513), (4224, 416, 640), (4160, 96, 300),
