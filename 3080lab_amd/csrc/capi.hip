@@ -617,6 +617,27 @@ static int launch_mmq_r_tg(const GemvArgs& a, hipStream_t s) {
   return -1;
 }
 
+// K slices of the products that add into fixed point, up to 255 tokens
+static int mmq_slices(int N, int K) {
+  const int KS = 384 / (N / 64), most = K / 128;
+  return KS < 1 || most < 1 ? 1 : KS < most ? KS : most;
+}
+
+// 49 (QKV: 33) to 255 tokens: slices of up to four blocks run in k_mmq_s32 (1536 x 1536 at 64 tokens 9.4 us against 12.3, at
+// 40 tokens 9.2 against 8.6). Longer ones (the down product) stay on the 16-token
+// kernels: a wave would run its 18 blocks one latency after another (1536 x 8960, 77 / 200 tokens: 25.5 / 48 us against
+// 23.5 / 41).
+static bool mmq_short_slices(const GemvArgs& a, int KS) { return (a.K / 32 + KS - 1) / KS <= 4; }
+template <int EPI>
+static int launch_mmq_s32(const GemvArgs& a, int KS, hipStream_t s) {
+  GemvArgs b = a;
+  b.mmq_chunk = (a.K / 32 + KS - 1) / KS;
+  const dim3 grid(a.N / 32, 1, (a.T + 31) / 32), block(S32_KW * 64);
+  if (a.T <= 64) hipLaunchKernelGGL((k_mmq_s32<EPI, true>), grid, block, 0, s, b);
+  else hipLaunchKernelGGL((k_mmq_s32<EPI, false>), grid, block, 0, s, b);
+  return launched("mmq");
+}
+
 template <int EPI>
 static int launch_mmq_tg(const GemvArgs& a, int KS, hipStream_t s) {
   if constexpr (EPI == EPI_SWIGLU) {
@@ -631,19 +652,12 @@ static int launch_mmq_tg(const GemvArgs& a, int KS, hipStream_t s) {
   if constexpr (EPI == EPI_STORE || EPI == EPI_RESID_FIX || EPI == EPI_SWIGLU_Q8)
     if ((a.N % 128 == 0 && (a.N / 128) * ((a.T + 63) / 64) >= 256) || (a.T >= 256 && (EPI != EPI_SWIGLU_Q8 || a.N % 128 == 0)))
       return launch_mmq_big<EPI>(a, s);
+  if constexpr (EPI == EPI_RESID_FIX)
+    if (a.T > 48 && mmq_short_slices(a, KS)) return launch_mmq_s32<EPI>(a, KS, s);
   // up to 64 tokens (decode batches): 16-token workgroups, several per CU, hide each other's latencies; what is left of
   // the larger calls: 32- or 64-token workgroups reuse every staged weight block 2 or 4 times
   if (a.T <= 64) return launch_mmq<1, EPI>(a, KS, s);
-  if constexpr (EPI == EPI_RESID_FIX) {                // 65 to 255 tokens
-    const int per = (a.K / 32 + KS - 1) / KS;
-    // longer slices (the down product) stay on the 16-token kernel: a wave would run its 18 blocks one latency after
-    // another (1536 x 8960, 77 / 200 tokens: 25.5 / 48 us against 23.5 / 41)
-    if (per > 4) return launch_mmq<2, EPI>(a, KS, s);
-    GemvArgs b = a;
-    b.mmq_chunk = per;
-    hipLaunchKernelGGL(k_mmq_s32, dim3(a.N / 32, 1, (a.T + 31) / 32), dim3(S32_KW * 64), 0, s, b);
-    return launched("mmq");
-  }
+  if constexpr (EPI == EPI_RESID_FIX) return launch_mmq<2, EPI>(a, KS, s);
   // STORE has no K split over the grid: 64 x 32 tiles of eight K waves, their fp32 chains added in f64 (us at 77 tokens,
   // k_mmq<2> with four: 1536 x 8960 25 against 56, 1536 x 1536 7.7 against 12.3)
   if constexpr (EPI == EPI_STORE) return launch_mmq_t32<2, 1, 1, 1, 8, EPI>(a, s);
@@ -660,7 +674,6 @@ extern "C" int q355_mmq_q4_0_q8_1(const uint8_t* qs, const void* d, int N, int K
   GemvArgs a = {};
   a.qs = qs; a.d = (const __half*)d; a.N = N; a.K = K; a.T = T; a.xq = xq; a.xds = (const half2*)xds;
   hipStream_t s = (hipStream_t)stream;
-  const int nb = K / 32, groups = N / 64;
   switch (epi) {
     case 0:
       REQUIRE(y, "mmq_q4_0_q8_1: store needs y");
@@ -669,9 +682,7 @@ extern "C" int q355_mmq_q4_0_q8_1(const uint8_t* qs, const void* d, int N, int K
     case 6: {
       REQUIRE(yfix, "mmq_q4_0_q8_1: resid_fix needs yfix");
       a.yfix = (long long*)yfix;
-      int KS = 384 / groups;                          // launch_mmq only: prefill sizes have parallelism enough
-      KS = KS < 1 ? 1 : (KS > nb / 4 ? nb / 4 : KS);
-      if (KS < 1) KS = 1;
+      const int KS = mmq_slices(N, K);                // up to 255 tokens: prefill sizes have parallelism enough
       return launch_mmq_tg<EPI_RESID_FIX>(a, KS, s);
     }
     case 4:
@@ -1040,8 +1051,8 @@ extern "C" int q355_qkv_finish(int64_t* acc, const float* bias, const float* rop
 }
 
 // QKV product with the finish fused into its epilogue: every output has one writer (no K split), so no int64
-// accumulator and no second launch. Decode batches (T <= 32, K <= 1536) run the register-resident kernel,
-// larger T the LDS-tiled one.
+// accumulator and no second launch. Decode batches (T <= 32, K <= 1536) run the register-resident kernel, 33 to 255
+// tokens over a short K k_mmq_s32, larger T k_mmq_t32.
 extern "C" int q355_mmq_qkv_rope(const uint8_t* qs, const void* d, int N, int K, const int8_t* xq, const void* xds,
                                  int T, const float* bias, const float* rope_cos, const float* rope_sin,
                                  const int32_t* pos, const int32_t* block_table, int bt_stride, int seq_stride,
@@ -1065,6 +1076,8 @@ extern "C" int q355_mmq_qkv_rope(const uint8_t* qs, const void* d, int N, int K,
                           : launch_mmq_r_tg<2, EPI_QKV, false>(a, (hipStream_t)stream);
     if (r >= 0) return r;
   }
+  const int KS = mmq_slices(N, K);
+  if (T < 256 && mmq_short_slices(a, KS)) return launch_mmq_s32<EPI_QKV>(a, KS, (hipStream_t)stream);
   return launch_mmq_big<EPI_QKV>(a, (hipStream_t)stream);
 }
 

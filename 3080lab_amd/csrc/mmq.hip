@@ -1059,9 +1059,9 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
   }
 }
 
-// RESID_FIX for 65 to 255 tokens over a short K (the qkv and o products), where the tiles are few: the K slices of
-// k_mmq_reg's grid (a.mmq_chunk <= 4 blocks each; the fp32 block terms of a slice added in f64 and rounded to fixed point:
-// the same bytes), but a slice is one wave's 32 x 32 tile, and the workgroup's waves take the slices of one tile and add
+// RESID_FIX (49 to 255 tokens) and QKV (33 to 255) over a short K (the o and qkv products), where the tiles are few: the K slices of
+// k_mmq_reg's grid (a.mmq_chunk <= 4 blocks each; the block terms of a slice, fp32 or up to 64 tokens exact in f64, added
+// in f64 and rounded to fixed point: the same bytes), but a slice is one wave's 32 x 32 tile, and the workgroup's waves take the slices of one tile and add
 // them through LDS, so an output has one writer: the int64 atomics of the slices (one per output and slice) had been
 // most of the time. A wave loads the blocks of two slices before its first product: one memory latency.
 // Measured (us at 77 / 150 / 250 tokens; k_mmq_reg with atomics before): 1536 x 1536 9.6 / 9.9 / 17.2 (11.8 / 20 / 31), 2048 x
@@ -1069,6 +1069,7 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
 // CU (registers) by their rounds.
 constexpr int S32_KW = 6;
 
+template <int EPI, bool F64>
 __global__ void __launch_bounds__(S32_KW * 64) k_mmq_s32(const GemvArgs a) {
   __shared__ unsigned long long part[16][64];
   const int K = a.K, nb = K / 32, N = a.N, per = a.mmq_chunk;
@@ -1114,7 +1115,10 @@ __global__ void __launch_bounds__(S32_KW * 64) k_mmq_s32(const GemvArgs a) {
               snib16(make_uint4(w[i][e].x, w[i][e].y, w[i][e].z, w[i][e].w), sh), x[i][e], zi, 0, 0, 0);
           const v16f sc = __builtin_amdgcn_mfma_f32_32x32x8f16(half0(dw[i][e] & lo), half0(dx[i][e] & lo), zf, 0, 0, 0);
 #pragma unroll
-          for (int v = 0; v < 16; ++v) s[v] += (double)(sc[v] * 0.0625f * (float)c[v]);
+          for (int v = 0; v < 16; ++v) {
+            if constexpr (F64) s[v] = fma((double)(sc[v] * 0.0625f), (double)c[v], s[v]);
+            else s[v] += (double)(sc[v] * 0.0625f * (float)c[v]);
+          }
         }
 #pragma unroll
       for (int v = 0; v < 16; ++v) sum[v] += to_fix(s[v]);
@@ -1128,12 +1132,38 @@ __global__ void __launch_bounds__(S32_KW * 64) k_mmq_s32(const GemvArgs a) {
   for (int e = tid; e < 512; e += S32_KW * 64) {                      // 2 consecutive rows of one token
     const int r = (e & 15) * 2, t = e >> 4;
     const int pv = 4 * (r >> 3) + (r & 3), pl = t + 32 * ((r >> 2) & 1);
-    if (tok0 + t < a.T) {
-      longlong2* y = (longlong2*)(a.yfix + (size_t)(tok0 + t) * N + row0 + r);
+    const int tk = tok0 + t, row = row0 + r;
+    if (tk >= a.T) continue;
+    const long long f0 = (long long)part[pv][pl], f1 = (long long)part[pv + 1][pl];
+    if constexpr (EPI == EPI_RESID_FIX) {
+      longlong2* y = (longlong2*)(a.yfix + (size_t)tk * N + row);
       longlong2 h = *y;
-      h.x += (long long)part[pv][pl];
-      h.y += (long long)part[pv + 1][pl];
+      h.x += f0;
+      h.y += f1;
       *y = h;
+    } else {                                                          // as k_qkv_finish: the two rows are a RoPE pair
+      const int nq = a.nh * HD, nk = a.nkv * HD, pos = a.pos[tk];
+      const int pg = a.block_table[(size_t)(tk * a.seq_stride) * a.bt_stride + pos / PAGE];
+      const double v0 = from_fix(f0) + (double)a.aux[row], v1 = from_fix(f1) + (double)a.aux[row + 1];
+      if (row < nq + nk) {
+        const int i = (row % HD) >> 1;
+        const double c = a.rope_cos[(size_t)pos * (HD / 2) + i], s = a.rope_sin[(size_t)pos * (HD / 2) + i];
+        const __half lh16 = half_rn(v0 * c - v1 * s), hh16 = half_rn(v1 * c + v0 * s);
+        __half* dst = row < nq ? a.qout + (size_t)tk * nq + (row / HD) * HD
+                               : a.kcache + (((size_t)pg * a.nkv + (row - nq) / HD) * PAGE + pos % PAGE) * HD;
+        dst[i] = lh16;
+        dst[i + HD / 2] = hh16;
+        if (row < nq && a.qout64) {
+          double* d64 = a.qout64 + (size_t)tk * nq + (row / HD) * HD;
+          d64[i] = (double)__half2float(lh16);
+          d64[i + HD / 2] = (double)__half2float(hh16);
+        }
+      } else {
+        const int rv = row - nq - nk;
+        __half* vd = a.vcache + (((size_t)pg * a.nkv + rv / HD) * PAGE + pos % PAGE) * HD + rv % HD;
+        vd[0] = half_rn(v0);
+        vd[1] = half_rn(v1);
+      }
     }
   }
 }

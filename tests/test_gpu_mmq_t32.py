@@ -10,6 +10,7 @@ import pytest
 from lab import qwen_model as QM
 from lab.hip import call, ptr
 from oracle import quant as OQ
+from test_gpu_prefill import test_mmq_qkv_rope_equals_finish as qkv_rope_equals_finish
 
 pytestmark = pytest.mark.gpu
 
@@ -40,10 +41,11 @@ def reference(wb, dw, xq, dx, N, K, T):
     return y, (nb + 1) * 2.0 ** -23 * mag
 
 
-# dispatch: 65 to 255 tokens: RESID_FIX slices of one tile per workgroup (k_mmq_s32), STORE eight K waves; then up to 4096
-# rows one 32 x 32 tile per wave, with four K waves from 256 to 511 tokens (128- or, for an odd multiple of 64 rows, 64-row
-# workgroups from 512); wider 256 x 32, 128 x 64 or 128 x 128 workgroups
-@pytest.mark.parametrize("N,K,T", [(64, 32, 65), (128, 288, 97), (1536, 160, 200), (192, 8960, 70), (4096, 96, 255),
+# dispatch: 49 to 255 tokens over a short K: RESID_FIX slices of one tile per workgroup (k_mmq_s32, f64 up to 64 tokens),
+# STORE from 65 tokens eight K waves; then up to 4096 rows one 32 x 32 tile per wave, with four K waves from 256 to 511
+# tokens (128- or, for an odd multiple of 64 rows, 64-row workgroups from 512); wider 256 x 32, 128 x 64 or 128 x 128
+@pytest.mark.parametrize("N,K,T", [(64, 32, 49), (128, 224, 64), (1536, 1536, 50), (64, 32, 65), (128, 288, 97),
+                                   (1536, 160, 200), (192, 8960, 70), (4096, 96, 255),
                                    (64, 32, 256), (128, 288, 257), (1536, 160, 333), (192, 96, 511), (4096, 64, 300),
                                    (128, 32, 512), (64, 96, 545), (192, 128, 513), (128, 160, 575),
                                    (128, 288, 576), (4096, 96, 513), (2048, 32, 1100),
@@ -92,3 +94,9 @@ def test_mmq_t32_swiglu_is_the_quantized_store(cuda, T):
     ds = ods.cpu().numpy().astype(np.float64)
     assert (np.abs(ds[..., 0] - d) <= 2.0 ** -10 * np.abs(d) + 2.0 ** -24).all()
     assert np.allclose(ds[..., 1], ds[..., 0] * oq.cpu().numpy().reshape(T, -1, 32).sum(2), rtol=2e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("T,seq_stride", [(33, 0), (64, 1), (65, 0), (255, 0), (256, 0), (511, 0), (512, 0)])
+def test_qkv_rope_forms(cuda, T, seq_stride):
+    """The fused QKV finish of every form (k_mmq_s32 in f64 and fp32, four K waves, one) against the split product."""
+    qkv_rope_equals_finish(cuda, T, seq_stride)
