@@ -510,25 +510,26 @@ static int device_cus() {
   return cus[dev];
 }
 
-template <int RT, int TN, int RW, int CW, int KW, int EPI>
+template <int RT, int TN, int RW, int CW, int KW, int CB, int EPI>
 static int launch_mmq_t32(const GemvArgs& a, hipStream_t s) {
-  using L = T32<RT, TN, RW, CW, KW>;
-  hipLaunchKernelGGL((k_mmq_t32<RT, TN, RW, CW, KW, EPI>), dim3(a.N / L::ROWS, 1, (a.T + L::TOKS - 1) / L::TOKS),
+  using L = T32<RT, TN, RW, CW, KW, CB>;
+  hipLaunchKernelGGL((k_mmq_t32<RT, TN, RW, CW, KW, CB, EPI>), dim3(a.N / L::ROWS, 1, (a.T + L::TOKS - 1) / L::TOKS),
                      dim3(L::NTH), L::LDS, s, a);
   return launched("mmq");
 }
 
 // Up to 4096 rows (the qkv, o and down products) the tiles are few, so each wave takes one 32 x 32 tile.
 // From 512 tokens a wave takes the whole K, whatever T is, so that a prompt prefilled in chunks of 512 tokens and more
-// gives the sums of one chunk. us at 512 / 1024 / 2048 tokens, 1536 x 8960: 59 / 76 / 102 (16x16x32 tiles 89 / 110 /
-// 135; 128 x 64 workgroups of 32 x 64 tiles 90 / 91 / 121); 1536 x 1536: 14.6 / 19.3 / 24.7; 2048 x 1536: 12.9 / 16.9 / 27.8.
-// 256 to 511 tokens: four K waves per tile (333 tokens: 1536 x 8960 45 us against 59 with one and 89 for k_mmq<4>,
-// whose sums these are; 1536 x 1536 11.8 against 14.3 and 19.8).
+// gives the sums of one chunk: up to two 64 x 64 workgroups per CU with chunks of 8 blocks (the wait for the next chunk is
+// what bounds them), more of them 128 x 32 with chunks of 4. us at 512 / 1024 / 2048 tokens, 1536 x 8960: 53 / 74 / 102
+// (the other form 59 / 77 / 114; 16x16x32 tiles 89 / 110 / 135); 1536 x 1536: 13.7 / 19.1 / 25; 2048 x 1536: 14.0 / 20.0 / 28.
+// 256 to 511 tokens: four K waves per tile, chunks of 8 (333 tokens: 1536 x 8960 35 us, 44 with chunks of 4, 89 for
+// k_mmq<4>, whose sums these are; 1536 x 1536 9.7, 11.5 and 19.8).
 template <int EPI>
 static int launch_mmq_narrow(const GemvArgs& a, hipStream_t s) {
-  if (a.T >= 256 && a.T < 512) return launch_mmq_t32<1, 1, 1, 1, 4, EPI>(a, s);
-  if (a.N % 128) return launch_mmq_t32<1, 1, 2, 2, 1, EPI>(a, s);
-  return launch_mmq_t32<1, 1, 4, 1, 1, EPI>(a, s);
+  if (a.T >= 256 && a.T < 512) return launch_mmq_t32<1, 1, 1, 1, 4, 8, EPI>(a, s);
+  if (a.N % 128 || (long)(a.N / 64) * ((a.T + 63) / 64) <= 2 * device_cus()) return launch_mmq_t32<1, 1, 2, 2, 1, 8, EPI>(a, s);
+  return launch_mmq_t32<1, 1, 4, 1, 1, 4, EPI>(a, s);
 }
 
 // Prefill sizes (STORE, RESID_FIX, SWIGLU_Q8, QKV): k_mmq_t32. Wide matrices take one wave per tile, so the summation
@@ -542,9 +543,9 @@ static int launch_mmq_big(const GemvArgs& a, hipStream_t s) {
   const long cu = device_cus();
   const auto full = [&](int rows, int toks) { return (double)(((long)a.N / rows * ((a.T + toks - 1) / toks) + cu - 1) / cu); };
   const double c1 = 10.8 + 7.2 * full(128, 64), c2 = 17 + 11 * full(128, 128), c3 = 12 + 8 * full(256, 32);
-  if (a.N % 256 == 0 && c3 < c1 && c3 < c2) return launch_mmq_t32<2, 1, 4, 1, 1, EPI>(a, s);
-  if (c2 <= c1) return launch_mmq_t32<2, 2, 2, 2, 1, EPI>(a, s);
-  return launch_mmq_t32<2, 1, 2, 2, 1, EPI>(a, s);
+  if (a.N % 256 == 0 && c3 < c1 && c3 < c2) return launch_mmq_t32<2, 1, 4, 1, 1, 4, EPI>(a, s);
+  if (c2 <= c1) return launch_mmq_t32<2, 2, 2, 2, 1, 4, EPI>(a, s);
+  return launch_mmq_t32<2, 1, 2, 2, 1, 4, EPI>(a, s);
 }
 
 // LOGITS over a large vocabulary (N % 128 == 0) for up to 64 tokens: the LDS-tiled kernel with all tokens
@@ -660,7 +661,7 @@ static int launch_mmq_tg(const GemvArgs& a, int KS, hipStream_t s) {
   if constexpr (EPI == EPI_RESID_FIX) return launch_mmq<2, EPI>(a, KS, s);
   // STORE has no K split over the grid: 64 x 32 tiles of eight K waves, their fp32 chains added in f64 (us at 77 tokens,
   // k_mmq<2> with four: 1536 x 8960 25 against 56, 1536 x 1536 7.7 against 12.3)
-  if constexpr (EPI == EPI_STORE) return launch_mmq_t32<2, 1, 1, 1, 8, EPI>(a, s);
+  if constexpr (EPI == EPI_STORE) return launch_mmq_t32<2, 1, 1, 1, 8, 8, EPI>(a, s);
   else return a.T < 256 ? launch_mmq<2, EPI>(a, KS, s) : launch_mmq<4, EPI>(a, KS, s);
 }
 

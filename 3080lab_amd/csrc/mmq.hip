@@ -750,9 +750,9 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
 // Measured (us, 2048 tokens; before: 16x16x32 products with fp32 scale products): 17920 x 1536 213 -> 160 in 128 x 128
 // workgroups (174 in 128 x 64), 1536 x 8960 135 -> 102, 1536 x 1536 32 -> 25 and 2048 x 1536 34 -> 28 in 128 x 32 ones of
 // a 32 x 32 tile per wave.
-template <int RT, int TN, int RW, int CW, int KW>
+// CB: K blocks per LDS chunk
+template <int RT, int TN, int RW, int CW, int KW, int CB>
 struct T32 {
-  static constexpr int CB = KW > 4 ? KW : 4;         // K blocks per LDS chunk
   static constexpr int NTH = RW * CW * KW * 64, ROWS = RW * RT * 32, TOKS = CW * TN * 32;
   static constexpr int BST = CB * 32 + 16;           // LDS bytes of one token's activations (padded: 16 rows cover all banks)
   static constexpr int XST = TOKS + 16;              // LDS floats of one block's activation scales
@@ -775,10 +775,10 @@ __device__ __forceinline__ v4i snib16(uint4 w, int sh) {
                (int)(((w.w << sh) & m) ^ f)};
 }
 
-template <int RT, int TN, int RW, int CW, int KW, int EPI>
+template <int RT, int TN, int RW, int CW, int KW, int CB, int EPI>
 __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a) {
-  using L = T32<RT, TN, RW, CW, KW>;
-  constexpr int CB = L::CB, NTH = L::NTH, ROWS = L::ROWS, TOKS = L::TOKS;
+  using L = T32<RT, TN, RW, CW, KW, CB>;
+  constexpr int NTH = L::NTH, ROWS = L::ROWS, TOKS = L::TOKS;
   constexpr int PA = ROWS * CB, PW = ROWS * CB / 8, PB = TOKS * CB * 2, PX = TOKS * CB;   // staged pieces per chunk
   static_assert((PA % NTH == 0 || PA <= NTH) && (PB % NTH == 0 || PB <= NTH) && PW <= NTH && (PX % NTH == 0 || PX <= NTH),
                 "staging shape");

@@ -1,5 +1,5 @@
 """The prefill products on 32 x 32 x 32 int8 tiles (k_mmq_t32) at the sizes where they can go wrong: K shorter than a
-staged chunk of 4 blocks, K that ends inside one, token counts around a tile, every tile form, activations of -128
+staged chunk of 4 or 8 blocks, K that ends inside one, token counts around a tile, every tile form, activations of -128
 and subnormal scales.
 
 Reference: the exact block dots with their scales, summed in float64. The kernel adds the nb exact terms of an output in
@@ -43,12 +43,12 @@ def reference(wb, dw, xq, dx, N, K, T):
 
 # dispatch: 49 to 255 tokens over a short K: RESID_FIX slices of one tile per workgroup (k_mmq_s32, f64 up to 64 tokens),
 # STORE from 65 tokens eight K waves; then up to 4096 rows one 32 x 32 tile per wave, with four K waves from 256 to 511
-# tokens (128- or, for an odd multiple of 64 rows, 64-row workgroups from 512); wider 256 x 32, 128 x 64 or 128 x 128
+# tokens (64 x 64 workgroups from 512, 128 x 32 past two per CU); wider 256 x 32, 128 x 64 or 128 x 128
 @pytest.mark.parametrize("N,K,T", [(64, 32, 49), (128, 224, 64), (1536, 1536, 50), (64, 32, 65), (128, 288, 97),
                                    (1536, 160, 200), (192, 8960, 70), (4096, 96, 255),
                                    (64, 32, 256), (128, 288, 257), (1536, 160, 333), (192, 96, 511), (4096, 64, 300),
                                    (128, 32, 512), (64, 96, 545), (192, 128, 513), (128, 160, 575),
-                                   (128, 288, 576), (4096, 96, 513), (2048, 32, 1100),
+                                   (128, 288, 576), (4096, 96, 513), (2048, 32, 1100), (4096, 288, 700),
                                    (4224, 32, 512), (4224, 160, 513), (4224, 416, 640), (4160, 96, 300),
                                    (17920, 96, 65), (17920, 32, 333)])
 def test_mmq_t32_store_and_resid(cuda, N, K, T):
