@@ -497,9 +497,10 @@ __global__ void __launch_bounds__(64) k_attn_merge(const AttnArgs a) {
 }
 
 // Merge of k_attn_batch_f64's split partials, f64, in split order: o = sum_s e^(M_s - M) o_s / sum_s
-// e^(M_s - M) L_s (M = max_s M_s). Workgroup (KV head, token), thread (head t / 64, dims 2 (t % 64), + 1):
-// the splits' (M, L) and two values are loaded in batches of up to SB splits (one memory latency each; a
-// later batch rescales the earlier sums to its maximum), then Q8_1 per 16-lane row (one 32-value block).
+// e^(M_s - M) L_s (M = max_s M_s). Thread (head t / 64, dims 2 (t % 64), + 1): lane s takes split s's (M, L) and its one
+// exponential (every lane computing all of them, up to 17 f64 exponentials of ~120 ns, had been most of the merge), which
+// the sums then read as scalars; the splits' values are loaded SB at a time (one memory latency each, the first beside
+// the (M, L)). Then Q8_1 per 16-lane row (one 32-value block). At most 64 splits (64 pages).
 // COH: the partials were written by other workgroups of the same launch (device-scope stores), so they are read
 // with device-scope loads; otherwise by an earlier launch, read with ordinary loads.
 template <int G, int SPG, int SB, bool COH>
@@ -513,31 +514,24 @@ __device__ __forceinline__ void merge_f64(const AttnArgs& a, const int kvh, cons
   auto ld2 = [&](size_t e) {                          // the double2 at P0 + e
     return COH ? __builtin_bit_cast(double2, coh.ld((unsigned)(e * 8))) : *(const double2*)(P0 + e);
   };
-  double M = -INFINITY, o0 = 0.0, o1 = 0.0, L = 0.0;
-  for (int s0 = 0; s0 < nsplit; s0 += SB) {             // one batch (one memory latency) up to SB splits
-    double2 ml[SB], x[SB];
+  const double2 ml = ld2(min(dp, nsplit - 1) * st + HD);
+  double M = 0.0, f = 0.0, o0 = 0.0, o1 = 0.0, L = 0.0;
+  for (int s0 = 0; s0 < nsplit; s0 += SB) {
+    double2 x[SB];
 #pragma unroll
     for (int s = 0; s < SB; ++s)
-      if (s0 + s < nsplit) {
-        ml[s] = ld2((s0 + s) * st + HD);
-        x[s] = ld2((s0 + s) * st + 2 * dp);
-      }
-    double Mb = M;
-#pragma unroll
-    for (int s = 0; s < SB; ++s)
-      if (s0 + s < nsplit) Mb = fmax(Mb, ml[s].x);
-    if (s0) {                                           // rescale the earlier batches to the new maximum
-      const double r = exp(M - Mb);
-      o0 *= r; o1 *= r; L *= r;
+      if (s0 + s < nsplit) x[s] = ld2((s0 + s) * st + 2 * dp);
+    if (s0 == 0) {
+      M = wave_max_d(ml.x);                           // the lanes past the last split repeat it
+      f = exp(ml.x - M);
     }
-    M = Mb;
 #pragma unroll
     for (int s = 0; s < SB; ++s)
       if (s0 + s < nsplit) {
-        const double f = exp(ml[s].x - M);
-        L = fma(f, ml[s].y, L);
-        o0 = fma(f, x[s].x, o0);
-        o1 = fma(f, x[s].y, o1);
+        const double fs = readlane_d(f, s0 + s);
+        L = fma(fs, readlane_d(ml.y, s0 + s), L);
+        o0 = fma(fs, x[s].x, o0);
+        o1 = fma(fs, x[s].y, o1);
       }
   }
   const float v0 = (float)(o0 / L), v1 = (float)(o1 / L);
@@ -879,13 +873,14 @@ __global__ void __launch_bounds__(64) k_attn_worklist(const int* __restrict__ po
   for (int i = base * nkv + t; i < cap; i += 64) work[i] = make_int4(-1, 0, 0, 0);
 }
 
-// The merge as its own launch: workgroup (KV head, token).
+// The merge as its own launch: one wave per (KV head, token, query head of the group), so that a batch's merges spread
+// over the chip (32 tokens, contexts U[256, 2048]: 4.8 us; one workgroup of G waves per (KV head, token), every lane with its own exponentials, 6.3).
 template <int G, int SPG>
-__global__ void __launch_bounds__(G * 64) k_attn_merge_f64(const AttnArgs a) {
+__global__ void __launch_bounds__(64) k_attn_merge_f64(const AttnArgs a) {
   const int kvh = blockIdx.x, j = blockIdx.y;
   const int nsplit = (a.pos[j] / PAGE + 1 + SPG - 1) / SPG;
   if (nsplit == 1) return;                              // finished by the attention kernel
-  merge_f64<G, SPG, 20, false>(a, kvh, j, nsplit, threadIdx.x);   // 20 splits (2 KB of context each) per load batch
+  merge_f64<G, SPG, 20, false>(a, kvh, j, nsplit, blockIdx.z * 64 + threadIdx.x);   // 20 splits per load batch
 }
 
 }  // namespace q355

@@ -735,7 +735,7 @@ static int launch_attn_f64(const AttnArgs& a, int T, hipStream_t s) {
     hipLaunchKernelGGL((k_attn_batch_f64<G, ATTN64_SPG>), dim3(a.nkv * nsp, T), dim3(ATTN64_SPG * 256), 0, s, a);
   if (int e = launched("attn_decode_f64")) return e;
   if (nsp == 1 || a.arrivals) return Q355_OK;          // every token fits one split, or merged by its last split
-  hipLaunchKernelGGL((k_attn_merge_f64<G, ATTN64_SPG>), dim3(a.nkv, T), dim3(G * 64), 0, s, a);
+  hipLaunchKernelGGL((k_attn_merge_f64<G, ATTN64_SPG>), dim3(a.nkv, T, G), dim3(64), 0, s, a);
   return launched("attn_merge_f64");
 }
 
