@@ -433,36 +433,45 @@ __global__ void __launch_bounds__(256) k_attn_merge_split(const AttnArgs a) {
 // Merge of the chunk partials of one (token, query head), f64, by ONE wave: lane c reads chunk c's
 // (m_c, l_c) and forms w_c = e^(m_c - M) (M = max_c m_c); lane l then sums dims 2l, 2l+1 of
 // sum_c w_c o_c in fixed chunk order (w_c broadcast from lane c) and divides by L = sum_c w_c l_c.
-// All loads of a group of 8 chunks are issued before their first use. nch <= 64.
+// nch <= 64.
 // The first batch of loads is clamped by maxc (the chunk slots the partials buffer holds), not by nch, so it
 // does not wait for the position; chunks past nch are masked to 0 (stale slots may hold anything).
 __device__ __forceinline__ void attn_merge_head(const double* __restrict__ P, int maxc, int nch, double* __restrict__ out) {
   const int lane = threadIdx.x & 63;
   const double* pc = P + (size_t)min(lane, maxc - 1) * (HD + 2);
   const double mc = pc[HD], lc = pc[HD + 1];
-  double2 v[8];
+  // the first 8 chunks do not wait for the position (nch); the rest of up to 32 follows in one go, so a context of 2048
+  // positions costs two memory latencies (at position 1811, four of 8 chunks each: the 8-layer step 253 us against 249)
+  constexpr int NV = 32;
+  double2 v[NV];
 #pragma unroll
   for (int u = 0; u < 8; ++u) v[u] = ((const double2*)(P + (size_t)min(u, maxc - 1) * (HD + 2)))[lane];
+#pragma unroll
+  for (int u0 = 8; u0 < NV; u0 += 8)
+    if (u0 < nch) {                                       // uniform
+#pragma unroll
+      for (int u = u0; u < u0 + 8; ++u) v[u] = ((const double2*)(P + (size_t)min(u, nch - 1) * (HD + 2)))[lane];
+    }
   const double M = wave_max_d(lane < nch ? mc : -INFINITY);
   const double w = lane < nch ? exp(mc - M) : 0.0;
   const double L = wave_sum_d(w * (lane < nch ? lc : 0.0));
-  const int2 wi = *reinterpret_cast<const int2*>(&w);
   double o0 = 0.0, o1 = 0.0;
-  for (int c0 = 0; c0 < nch; c0 += 8) {
+  for (int c0 = 0; c0 < nch; c0 += NV) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      int2 bi;
-      bi.x = __builtin_amdgcn_readlane(wi.x, c0 + u);   // 0 for chunks >= nch (w = 0 there)
-      bi.y = __builtin_amdgcn_readlane(wi.y, c0 + u);
-      const double wc = *reinterpret_cast<const double*>(&bi);
-      const bool live = c0 + u < nch;
-      o0 = fma(wc, live ? v[u].x : 0.0, o0);
-      o1 = fma(wc, live ? v[u].y : 0.0, o1);
-    }
-    if (c0 + 8 < nch) {
+    for (int u0 = 0; u0 < NV; u0 += 8)
+      if (c0 + u0 < nch) {                                // uniform
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        v[u] = ((const double2*)(P + (size_t)min(c0 + 8 + u, nch - 1) * (HD + 2)))[lane];
+        for (int u = u0; u < u0 + 8; ++u) {
+          const double wc = readlane_d(w, c0 + u);        // 0 for chunks >= nch (w = 0 there)
+          const bool live = c0 + u < nch;
+          o0 = fma(wc, live ? v[u].x : 0.0, o0);
+          o1 = fma(wc, live ? v[u].y : 0.0, o1);
+        }
+      }
+    if (c0 + NV < nch) {
+#pragma unroll
+      for (int u = 0; u < NV; ++u)
+        v[u] = ((const double2*)(P + (size_t)min(c0 + NV + u, nch - 1) * (HD + 2)))[lane];
     }
   }
   ((double2*)out)[lane] = make_double2(o0 / L, o1 / L);
