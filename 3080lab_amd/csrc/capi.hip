@@ -548,20 +548,16 @@ static int launch_mmq_big(const GemvArgs& a, hipStream_t s) {
   return launch_mmq_t32<2, 1, 2, 2, 1, 4, EPI>(a, s);
 }
 
-// LOGITS over a large vocabulary (N % 128 == 0) for up to 64 tokens: the LDS-tiled kernel with all tokens
-// in one workgroup, so each weight is read once (128 rows x 16 / 32 / 64 tokens per workgroup).
+// LOGITS over a large vocabulary (N % 128 == 0) for up to 64 tokens: the LDS-tiled kernels with 128 rows and all tokens
+// in one workgroup, so each weight is read once. Up to 16 tokens k_mmq_tile (16-token MFMAs: no work for padding), above
+// that k_mmq_t32, whose fp32 sums are the same bits (151936 x 1536, us at 16 / 24 / 32 / 48 / 64 tokens: k_mmq_tile 31 / 43 /
+// 43 / 66 / 67, k_mmq_t32 36 / 36 / 36 / 53 / 54; chunks of 8 blocks 58 at 32 tokens and 66 at 64: half the workgroups per
+// CU; two K waves per tile 34 and 61).
 static int launch_mmq_logits_tile(const GemvArgs& a, hipStream_t s) {
-  const dim3 grid(a.N / 128, 1, 1);
-  if (a.T <= 16) {
-    constexpr size_t lds = 2 * LdsTile<2, 1, 1, TILE_CB>::BUF;
-    hipLaunchKernelGGL((k_mmq_tile<2, 1, 1>), grid, dim3(128), lds, s, a);
-  } else if (a.T <= 32) {
-    constexpr size_t lds = 2 * LdsTile<2, 2, 1, TILE_CB>::BUF;
-    hipLaunchKernelGGL((k_mmq_tile<2, 2, 1>), grid, dim3(256), lds, s, a);
-  } else {
-    constexpr size_t lds = 2 * LdsTile<2, 2, 2, TILE_CB>::BUF;
-    hipLaunchKernelGGL((k_mmq_tile<2, 2, 2>), grid, dim3(256), lds, s, a);
-  }
+  if (a.T > 32) return launch_mmq_t32<2, 1, 2, 2, 1, 4, EPI_LOGITS>(a, s);
+  if (a.T > 16) return launch_mmq_t32<2, 1, 2, 1, 1, 4, EPI_LOGITS>(a, s);
+  constexpr size_t lds = 2 * LdsTile<2, TILE_CB>::BUF;
+  hipLaunchKernelGGL(k_mmq_tile<2>, dim3(a.N / 128, 1, 1), dim3(128), lds, s, a);
   return launched("mmq");
 }
 

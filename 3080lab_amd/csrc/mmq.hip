@@ -1,5 +1,5 @@
-// Q4_0 x Q8_1 matrix product on int8 MFMA (v_mfma_i32_16x16x32_i8), gfx950: batched decode
-// (T = 5..32 tokens per launch) and prefill (T up to 64 per launch, grid.z over token groups).
+// Q4_0 x Q8_1 matrix product on int8 MFMA, gfx950: batched decode (up to 64 tokens) and short prompts on
+// v_mfma_i32_16x16x32_i8, prefill and the head of more than 16 tokens on v_mfma_i32_32x32x32_i8 (k_mmq_t32, k_mmq_s32).
 //
 // One Q4_0 block (k = 32) of one 16-row tile against 16 tokens is exactly one MFMA: A = the tile's
 // weights as int8 16 (q - 8), B = the tokens' int8 activations, C = 16 x the exact int32 block dots
@@ -557,8 +557,8 @@ __global__ void __launch_bounds__(NW * 64) k_mmq_reg(const GemvArgs a) {
   Q355_TRACE_POINT(5);
 }
 
-// LM head of a decode batch (up to 64 tokens): a workgroup computes (RW * 64 rows) x (CW * 16 TG tokens) with RW x CW waves,
-// each wave a 64 x 16 TG sub-tile (4 row tiles x TG token groups, 4 TG MFMAs per K block) over the full K slice.
+// LM head of a decode batch of up to 16 tokens: a workgroup computes (RW * 64 rows) x 16 tokens with RW waves,
+// each wave a 64 x 16 sub-tile (4 row tiles, 4 MFMAs per K block) over the full K slice.
 // K advances in chunks of CB blocks staged in LDS, double-buffered: the global loads of chunk c + 1 are
 // issued (16 B per lane, contiguous) before chunk c is computed, and written to the other buffer after.
 // The weights enter the MFMA as signed int8 16 (q - 8): nibble moved to the high half of the byte with its
@@ -568,25 +568,25 @@ __global__ void __launch_bounds__(NW * 64) k_mmq_reg(const GemvArgs a) {
 // contiguous, conflict-free 512 B wave read):
 //   A  [RW*4 tiles][CB][16 rows][16 B]     nibbles as stored in HBM
 //   W  [RW*4 tiles][CB][16]                row scales (fp32)
-//   B  [CW*TG groups][CB][16 tokens][32 B] int8 activations; tokens 8..15 of a group swap their 16 B
+//   B  [CB][16 tokens][32 B]               int8 activations; tokens 8..15 swap their 16 B
 //                                          halves, so the two half-wave reads of a B operand use all banks
-//   X  [CB][CW*16*TG]                      activation scale / 16 (fp32)
+//   X  [CB][16]                            activation scale / 16 (fp32)
 // Epilogue from registers: fp32 logits and one (max, row) partial per 64 rows and token, the layout of the other LOGITS
 // kernels.
-template <int RW, int CW, int TG, int CB>
+template <int RW, int CB>
 struct LdsTile {
-  static constexpr int TW = CW * 16 * TG;            // tokens per workgroup
-  static constexpr int A = RW * 4 * CB * 256, W = RW * 4 * CB * 64, B = CW * TG * CB * 512;
+  static constexpr int TW = 16;                      // tokens per workgroup
+  static constexpr int A = RW * 4 * CB * 256, W = RW * 4 * CB * 64, B = CB * 512;
   static constexpr int X = CB * TW * 4;
   static constexpr int BUF = A + W + B + X;
 };
 
-template <int RW, int CW, int TG>
+template <int RW>
 __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
   constexpr int CB = TILE_CB;
-  using L = LdsTile<RW, CW, TG, CB>;
+  using L = LdsTile<RW, CB>;
   constexpr int TW = L::TW;
-  constexpr int NTH = RW * CW * 64;                  // threads
+  constexpr int NTH = RW * 64;                       // threads
   constexpr int NA = RW * 4 * CB * 16;               // 16-byte pieces of A per chunk
   constexpr int NWp = RW * 4 * CB * 2;               // of W (fp16 in HBM)
   constexpr int NBp = TW * CB * 2;                   // of B (two per token and block)
@@ -596,7 +596,6 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
   const KSlice ks(nb);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
-  const int wr = wv / CW, wc = wv % CW;              // this wave's row block and token block
   const int tile0 = blockIdx.x * RW * 4;             // first 16-row tile of the workgroup
   const int tok0 = blockIdx.z * TW;                  // first token of the workgroup
   const int tid = threadIdx.x;
@@ -646,13 +645,11 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
     }                                                                                             \
   }
 
-  float acc[4][TG][4];
+  float acc[4][4];
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int g = 0; g < TG; ++g)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[t][g][v] = 0.f;
+    for (int v = 0; v < 4; ++v) acc[t][v] = 0.f;
 
   int buf = 0;
   if (ks.b0 < ks.b1) {
@@ -664,35 +661,31 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
     const bool more = c0 + CB < ks.b1;               // uniform
     if (more) Q355_TILE_LOAD(c0 + CB);
     const char* base = lds + buf * L::BUF;
-    const char* sA = base + (size_t)(wr * 4) * CB * 256;
-    const char* sW = base + L::A + (size_t)(wr * 4) * CB * 64;
-    const char* sB = base + L::A + L::W + (size_t)(wc * TG) * CB * 512;
-    const float* sX = (const float*)(base + L::A + L::W + L::B) + wc * 16 * TG;
+    const char* sA = base + (size_t)(wv * 4) * CB * 256;
+    const char* sW = base + L::A + (size_t)(wv * 4) * CB * 64;
+    const char* sB = base + L::A + L::W;
+    const float* sX = (const float*)(base + L::A + L::W + L::B);
 #pragma unroll 1
     for (int blk = 0; blk < CB; ++blk) {
       long w[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) w[t] = snib8(*(const uint2*)(sA + (t * CB + blk) * 256 + li * 16 + (lg & 1) * 8), lg);
-      // the block scales d_w d_x of all 4 x 16 x 16 outputs of a token group in ONE 4-block outer product on
+      // the block scales d_w d_x of all 4 x 16 x 16 outputs in ONE 4-block outer product on
       // the matrix cores (v_mfma_f32_16x16x1f32: block t = tile t; lane 16 t + r supplies d_w of row r, every
       // lane d_x of its token li; lane l receives d_w[t][4 lg + v] d_x[li] in register 4 t + v): the 16
       // exact fp32 products that would otherwise be 16 VALU multiplies
       const float wl = *(const float*)(sW + (lg * CB + blk) * 64 + li * 4);
+      const long bx = *(const long*)(sB + (blk * 16 + li) * 32 + (lg ^ ((li >> 3) << 1)) * 8);
+      const v4i zero = {0, 0, 0, 0};
+      const v16f zf = {};
+      const v16f sc = __builtin_amdgcn_mfma_f32_16x16x1f32(wl, sX[blk * TW + li], zf, 0, 0, 0);
+      v4i c[4];
 #pragma unroll
-      for (int g = 0; g < TG; ++g) {
-        const long bx = *(const long*)(sB + ((g * CB + blk) * 16 + li) * 32 + (lg ^ ((li >> 3) << 1)) * 8);
-        const float dx = sX[blk * TW + g * 16 + li];
-        const v4i zero = {0, 0, 0, 0};
-        const v16f zf = {};
-        const v16f sc = __builtin_amdgcn_mfma_f32_16x16x1f32(wl, dx, zf, 0, 0, 0);
-        v4i c[4];
+      for (int t = 0; t < 4; ++t) c[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(w[t], bx, zero, 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) c[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(w[t], bx, zero, 0, 0, 0);
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) acc[t][g][v] = fmaf(sc[4 * t + v], (float)c[t][v], acc[t][g][v]);
-      }
+        for (int v = 0; v < 4; ++v) acc[t][v] = fmaf(sc[4 * t + v], (float)c[t][v], acc[t][v]);
     }
     if (more) {
       Q355_TILE_STORE(buf ^ 1);
@@ -703,34 +696,31 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
 #undef Q355_TILE_LOAD
 #undef Q355_TILE_STORE
 
-  const int rt0 = tile0 + wr * 4;                    // this wave's first row tile
+  const int rt0 = tile0 + wv * 4;                    // this wave's first row tile
+  const int tok = tok0 + li;
+  const bool ok = tok < a.T;
+  // fp32 logits, and this wave's (max, lowest row) over its 64 rows: partial rt0 / 4 of N / 64
+  float bv = -INFINITY;
+  int bi = 0x7fffffff;
 #pragma unroll
-  for (int g = 0; g < TG; ++g) {
-    const int tok = tok0 + wc * 16 * TG + g * 16 + li;
-    const bool ok = tok < a.T;
-    // fp32 logits, and this wave's (max, lowest row) over its 64 rows: partial rt0 / 4 of N / 64
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
+  for (int t = 0; t < 4; ++t) {
+    if (ok && a.y)                                     // fp32 logits are optional: the argmax needs only partials
+      *(float4*)(a.y + (size_t)tok * N + (rt0 + t) * 16 + 4 * lg) =
+          make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      if (ok && a.y)                                     // fp32 logits are optional: the argmax needs only partials
-        *(float4*)(a.y + (size_t)tok * N + (rt0 + t) * 16 + 4 * lg) =
-            make_float4(acc[t][g][0], acc[t][g][1], acc[t][g][2], acc[t][g][3]);
+    for (int v = 0; v < 4; ++v)                        // rows increase with (t, v): strict '>' keeps the lowest
+      if (acc[t][v] > bv) { bv = acc[t][v]; bi = (rt0 + t) * 16 + 4 * lg + v; }
+  }
 #pragma unroll
-      for (int v = 0; v < 4; ++v)                        // rows increase with (t, v): strict '>' keeps the lowest
-        if (acc[t][g][v] > bv) { bv = acc[t][g][v]; bi = (rt0 + t) * 16 + 4 * lg + v; }
-    }
-#pragma unroll
-    for (int o = 16; o <= 32; o <<= 1) {
-      const float ov = __shfl_xor(bv, o);
-      const int oi = __shfl_xor(bi, o);
-      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-    }
-    if (ok && lg == 0) {
-      const int np = N / 64;
-      a.pmax[(size_t)tok * np + rt0 / 4] = bv;
-      a.pidx[(size_t)tok * np + rt0 / 4] = bi;
-    }
+  for (int o = 16; o <= 32; o <<= 1) {
+    const float ov = __shfl_xor(bv, o);
+    const int oi = __shfl_xor(bi, o);
+    if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+  }
+  if (ok && lg == 0) {
+    const int np = N / 64;
+    a.pmax[(size_t)tok * np + rt0 / 4] = bv;
+    a.pidx[(size_t)tok * np + rt0 / 4] = bi;
   }
 }
 
@@ -749,7 +739,8 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
 // the VALU up: converts do not overlap with them. Counters at 17920 x 1536 x 2048 tokens: VALU 84 % busy.
 // Measured (us, 2048 tokens; before: 16x16x32 products with fp32 scale products): 17920 x 1536 213 -> 160 in 128 x 128
 // workgroups (174 in 128 x 64), 1536 x 8960 135 -> 102, 1536 x 1536 32 -> 25 and 2048 x 1536 34 -> 28 in 128 x 32 ones of
-// a 32 x 32 tile per wave.
+// a 32 x 32 tile per wave. The tied head (151936 x 1536, LOGITS) at 24 and 32 tokens 43 -> 36 in 128 x 32 workgroups of two
+// waves, at 64 tokens 67 -> 54 in 128 x 64: there the wait for the next chunk bounds it (131 MB would take 25).
 // CB: K blocks per LDS chunk
 template <int RT, int TN, int RW, int CW, int KW, int CB>
 struct T32 {
@@ -1000,6 +991,35 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
         const int Nout = N / 2, ob = tile0 / 4 + wr;   // output Q8_1 block of this wave's 64 rows
         *(uint4*)(a.oq + (size_t)tok * Nout + ob * 32 + 16 * lh) = make_uint4(word[0], word[1], word[2], word[3]);
         if (!lh) a.ods[(size_t)tok * (Nout / 32) + ob] = __halves2half2(__float2half_rn(d32), q8_s16(d32, sq));
+      }
+    }
+    return;
+  }
+  if constexpr (EPI == EPI_LOGITS) {
+    // fp32 logits (optional: the argmax needs only partials), and this wave's (max, lowest row) over its 64 rows: partial
+    // tile0 / 4 + wr of N / 64, the layout of the other LOGITS kernels
+    static_assert(EPI != EPI_LOGITS || (RT == 2 && KW == 1), "64 rows per wave");
+#pragma unroll
+    for (int g = 0; g < TN; ++g) {
+      const int tok = tokb + 32 * g;
+      const bool ok = tok < a.T;
+      float bv = -INFINITY;
+      int bi = 0x7fffffff;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int row = rowb + 8 * i;                    // 32 (i / 4) + 8 (i % 4)
+        const auto& s = sum[g * 8 + i];
+        if (ok && a.y) *(float4*)(a.y + (size_t)tok * N + row) = make_float4(s[0], s[1], s[2], s[3]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)                      // rows increase with (i, e): strict '>' keeps the lowest
+          if (s[e] > bv) { bv = s[e]; bi = row + e; }
+      }
+      const float ov = __shfl_xor(bv, 32);
+      const int oi = __shfl_xor(bi, 32);
+      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+      if (ok && !lh) {
+        a.pmax[(size_t)tok * (N / 64) + tile0 / 4 + wr] = bv;
+        a.pidx[(size_t)tok * (N / 64) + tile0 / 4 + wr] = bi;
       }
     }
     return;

@@ -69,6 +69,31 @@ def test_mmq_t32_store_and_resid(cuda, N, K, T):
     assert (np.abs(got - ref) <= bound + 2.0 ** -48).all()
 
 
+# the tied head of a batch: 16-token tiles up to 16 tokens, 128 x 32 up to 32, 128 x 64 up to 64
+@pytest.mark.parametrize("K,T", [(32, 1), (160, 16), (32, 17), (160, 31), (288, 32), (96, 33), (1536, 63), (128, 64)])
+def test_logits_and_their_partials(cuda, K, T):
+    """Logits within the bound; every (max, lowest row) over 64 rows is that of the stored logits, also without them."""
+    import torch
+    N = 128 * 256 + 128
+    wb, dw, xq, dx = problem(N, K, T, K + T)
+    W = QM.Q4Mat(wb, N, K, "cuda")
+    xq_d = torch.from_numpy(xq).cuda()
+    xds_d = torch.from_numpy(np.stack([dx, np.zeros_like(dx)], -1)).cuda()
+    ref, bound = reference(wb, dw, xq, dx, N, K, T)
+    y = torch.full((T, N), float("nan"), device=cuda)
+    for out in (ptr(y), None):
+        pmax = torch.full((T, N // 64), float("nan"), device=cuda)
+        pidx = torch.full((T, N // 64), -1, dtype=torch.int32, device=cuda)
+        call("q355_mmq_q4_0_q8_1", ptr(W.qs), ptr(W.d), N, K, ptr(xq_d), ptr(xds_d), T, 5, out, None, None, None, ptr(pmax),
+             ptr(pidx))
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        tiles = got.reshape(T, N // 64, 64)
+        np.testing.assert_array_equal(pmax.cpu().numpy(), tiles.max(axis=2))
+        np.testing.assert_array_equal(pidx.cpu().numpy(), tiles.argmax(axis=2) + 64 * np.arange(N // 64))
+    assert (np.abs(got - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("T", [512, 577, 1100])
 def test_mmq_t32_swiglu_is_the_quantized_store(cuda, T):
     """SWIGLU_Q8 gives the Q8_1 rule of silu(g) u: codes within one step of those of the STORE sums, and d equal to the
