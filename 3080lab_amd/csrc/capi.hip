@@ -578,6 +578,8 @@ static void launch_mmq_r(const GemvArgs& a, dim3 grid, hipStream_t s) {
   hipLaunchKernelGGL((k_mmq_r<TG, NT, NW, KPW, EPI, XF32>), grid, dim3(NW * 64), 0, s, a);
 }
 
+static bool mmq_qkv_in_registers(int N, int K) { return N % 16 == 0 && K <= 16 * 3 * 32; }
+
 template <int TG, int EPI, bool XF32>
 static int launch_mmq_r_tg(const GemvArgs& a, hipStream_t s) {
   const int nb = a.K / 32;
@@ -593,7 +595,7 @@ static int launch_mmq_r_tg(const GemvArgs& a, hipStream_t s) {
     // one writer per output (no K split): 16-row workgroups of 16 waves x 3 blocks (8 waves x 6: 5.77 / 9.80 us
     // at B = 8 / 32 against 5.20 / 8.94), bias + RoPE + K/V write in the epilogue (a RoPE pair sits in
     // adjacent rows of one tile)
-    if (a.N % 16 || nb > 16 * 3) return -1;
+    if (!mmq_qkv_in_registers(a.N, a.K)) return -1;
     launch_mmq_r<TG, 1, 16, 3, EPI, XF32>(a, dim3(a.N / 16), s);
     return launched("mmq");
   }
@@ -624,7 +626,7 @@ static int mmq_slices(int N, int K) {
 // 40 tokens 9.2 against 8.6). Longer ones (the down product) stay on the 16-token
 // kernels: a wave would run its 18 blocks one latency after another (1536 x 8960, 77 / 200 tokens: 25.5 / 48 us against
 // 23.5 / 41).
-static bool mmq_short_slices(const GemvArgs& a, int KS) { return (a.K / 32 + KS - 1) / KS <= 4; }
+static bool mmq_short_slices(int K, int KS) { return (K / 32 + KS - 1) / KS <= 4; }
 template <int EPI>
 static int launch_mmq_s32(const GemvArgs& a, int KS, hipStream_t s) {
   GemvArgs b = a;
@@ -650,7 +652,7 @@ static int launch_mmq_tg(const GemvArgs& a, int KS, hipStream_t s) {
     if ((a.N % 128 == 0 && (a.N / 128) * ((a.T + 63) / 64) >= 256) || (a.T >= 256 && (EPI != EPI_SWIGLU_Q8 || a.N % 128 == 0)))
       return launch_mmq_big<EPI>(a, s);
   if constexpr (EPI == EPI_RESID_FIX)
-    if (a.T > 48 && mmq_short_slices(a, KS)) return launch_mmq_s32<EPI>(a, KS, s);
+    if (a.T > 48 && mmq_short_slices(a.K, KS)) return launch_mmq_s32<EPI>(a, KS, s);
   // up to 64 tokens (decode batches): 16-token workgroups, several per CU, hide each other's latencies; what is left of
   // the larger calls: 32- or 64-token workgroups reuse every staged weight block 2 or 4 times
   if (a.T <= 64) return launch_mmq<1, EPI>(a, KS, s);
@@ -1047,6 +1049,14 @@ extern "C" int q355_qkv_finish(int64_t* acc, const float* bias, const float* rop
   return launched("qkv_finish");
 }
 
+// The fused product of up to this many tokens (below 256) sums as precisely as the split form, the RESID_FIX product and
+// q355_qkv_finish: in f64 (up to 32 tokens, the whole K in registers), or over the same slices (k_mmq_s32). Elsewhere
+// below 256 tokens it is one fp32 chain over the whole K (k_mmq_t32), where the split form adds f64 or short slices.
+extern "C" int q355_mmq_qkv_fused_max_t(int N, int K) {
+  if (N < 64 || N % 64 || K < 32 || K % 32) return 0;
+  return mmq_short_slices(K, mmq_slices(N, K)) ? 255 : mmq_qkv_in_registers(N, K) ? 32 : 0;
+}
+
 // QKV product with the finish fused into its epilogue: every output has one writer (no K split), so no int64
 // accumulator and no second launch. Decode batches (T <= 32, K <= 1536) run the register-resident kernel, 33 to 255
 // tokens over a short K k_mmq_s32, larger T k_mmq_t32.
@@ -1074,7 +1084,7 @@ extern "C" int q355_mmq_qkv_rope(const uint8_t* qs, const void* d, int N, int K,
     if (r >= 0) return r;
   }
   const int KS = mmq_slices(N, K);
-  if (T < 256 && mmq_short_slices(a, KS)) return launch_mmq_s32<EPI_QKV>(a, KS, (hipStream_t)stream);
+  if (T < 256 && mmq_short_slices(K, KS)) return launch_mmq_s32<EPI_QKV>(a, KS, (hipStream_t)stream);
   return launch_mmq_big<EPI_QKV>(a, (hipStream_t)stream);
 }
 

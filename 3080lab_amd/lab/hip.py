@@ -63,6 +63,7 @@ _SIGS = {
     "q355_qkv_finish": [_P, _P, _P, _P, _P, _P, c_int, c_int, _P, _P, _P, c_int, c_int, c_int, _P],
     "q355_mmq_qkv_rope": [_P, _P, c_int, c_int, _P, _P, c_int, _P, _P, _P, _P, _P, c_int, c_int, _P, _P, _P, _P,
                           c_int, c_int, _P],
+    "q355_mmq_qkv_fused_max_t": [c_int, c_int],
     "q355_attn_decode_f64": [_P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_double, _P, _P, _P, _P, c_int, _P],
     "q355_attn_decode_f64_wl": [_P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_double, _P, _P, _P, _P, c_int, _P,
                                 _P],
@@ -73,7 +74,7 @@ _SIGS = {
                                c_int, c_int, _P],
 }
 # entry points returning something other than an int status
-_VALUE_FUNCS = {"q355_attn_decode_noalloc_max_bytes", "q355_head_nparts", "q355_mmq_nparts", "q355_mega_ws_bytes", "q355_mega_layer_bytes",
+_VALUE_FUNCS = {"q355_attn_decode_noalloc_max_bytes", "q355_head_nparts", "q355_mmq_nparts", "q355_mmq_qkv_fused_max_t", "q355_mega_ws_bytes", "q355_mega_layer_bytes",
                 "q355_attn_prefill_ws_bytes", "q355_attn_f64_worklist_bytes"}
 
 _lib = None

@@ -302,16 +302,15 @@ def flash_prefill_v3_source(maxlen: int = 4096, q8: bool = True) -> KernelSpec:
 
 
 # chunks of at least this many tokens, and short ones, run the QKV product with the finish in its epilogue
-# (q355_mmq_qkv_rope: one launch, no int64 accumulator; 77 tokens: 10 us against 16.5 + 5.4, 333 tokens: 12 against 24 +
-# 6). Short is up to 32 tokens (register-resident, f64), or up to 255 where the product's K slices are of up to four
-# blocks (the same fixed-point sums as the split form). The others keep the K-split product into the int64 accumulator
-# plus q355_qkv_finish. From 512 tokens on no product's summation order depends on the chunk, so chunking a prompt into
-# pieces of >= 512 tokens gives the same results bit for bit.
+# (q355_mmq_qkv_rope: one launch, no int64 accumulator; 2048 x 1536 at 77 tokens: 10 us against 16.5 + 5.4, at 333 tokens:
+# 12 against 24 + 6). Short is what the library says it sums as precisely as the split form (qkv_fused_small_p). The others
+# keep the K-split product into the int64 accumulator plus q355_qkv_finish. From 512 tokens on no product's summation
+# order depends on the chunk, so chunking a prompt into pieces of >= 512 tokens gives the same results bit for bit.
 QKV_FUSED_MIN_P = 256
 
 
 def qkv_fused_small_p(N: int, K: int) -> int:
-    return 255 if (K // 128) * (N // 64) <= 384 else 32
+    return call("q355_mmq_qkv_fused_max_t", N, K)
 
 
 class Prefill:
@@ -319,7 +318,7 @@ class Prefill:
 
     chunk(ids, pos0) runs P prompt tokens at positions pos0 .. pos0 + P - 1 through all layers at once:
       embed -> per layer: rmsnorm_fix_q8_1, MMQ qkv with bias + RoPE + K/V write in its epilogue
-      (P >= QKV_FUSED_MIN_P or P <= qkv_fused_small_p; else MMQ qkv into an int64 accumulator + qkv_finish),
+      (P >= QKV_FUSED_MIN_P or P <= qkv_fused_small_p(); else MMQ qkv into an int64 accumulator + qkv_finish),
       attn_prefill_q8_1 (causal, fp16 MFMA, Q8_1 output), MMQ o (+= h), rmsnorm_fix_q8_1, MMQ gate_up (SwiGLU -> Q8_1),
       MMQ down (+= h) -> final norm + head on the last token -> dec.tok = argmax, dec.pos = pos0 + P.
     The decoder then continues greedy decode from that state."""
@@ -329,6 +328,7 @@ class Prefill:
         m, c = dec.m, dec.cfg
         assert dec.T == 1, "prefill fills sequence 0 of a batch-1 decoder"
         self.dec, self.m, self.cfg, self.P_max = dec, m, c, max_chunk
+        self.qkv_small_p = qkv_fused_small_p(c.nqkv, c.H)
         dev = m.device
         P, H = max_chunk, c.H
         self.h = torch.zeros(P, H, dtype=torch.int64, device=dev)
@@ -351,7 +351,7 @@ class Prefill:
         L = m.layers[i]
         call("q355_rmsnorm_fix_q8_1", ptr(self.h), ptr(L["ln1"]), ptr(self.xq), ptr(self.xds), P, c.H, c.eps)
         W = L["qkv"]
-        if P >= QKV_FUSED_MIN_P or P <= qkv_fused_small_p(W.N, W.K):
+        if P >= QKV_FUSED_MIN_P or P <= self.qkv_small_p:
             # one writer per output: the finish (bias, RoPE, K/V write) runs in the GEMM epilogue
             call("q355_mmq_qkv_rope", ptr(W.qs), ptr(W.d), W.N, W.K, ptr(self.xq), ptr(self.xds), P, ptr(L["qkv_b"]),
                  ptr(m.cos), ptr(m.sin), ptr(self.pos), ptr(d.block_table), d.max_chunks, 0, ptr(d.kc[i]),

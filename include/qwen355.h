@@ -274,6 +274,11 @@ int q355_mmq_qkv_rope(const uint8_t* qs, const void* d, int N, int K, const int8
                       const int32_t* block_table, int bt_stride, int seq_stride, void* kcache, void* vcache,
                       void* qout, double* q64, int nh, int nkv, void* stream);
 
+/* Largest T below 256 for which q355_mmq_qkv_rope sums as precisely as q355_mmq_q4_0_q8_1 (epi 6) followed by
+ * q355_qkv_finish (0: none; from 256 tokens on it always does). Other calls of fewer than 256 tokens add the whole K in
+ * one fp32 chain. No counterpart in the reference. */
+int q355_mmq_qkv_fused_max_t(int N, int K);
+
 /* Batched decode attention of the int8 path, in f64 (the batch-1 arithmetic: f64 scores, softmax and P.V of
  * the fp16 q/K/V): T tokens, token j attends to positions 0 .. pos[j] of its paged K/V (block_table row j).
  * q64 [T][nh*128] f64 (q355_mmq_qkv_rope's q64). Splits of 2 pages, 4 waves per page, the GQA group's query
