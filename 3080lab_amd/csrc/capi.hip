@@ -523,12 +523,12 @@ static int launch_mmq_t32(const GemvArgs& a, hipStream_t s) {
 // gives the sums of one chunk: up to two 64 x 64 workgroups per CU with chunks of 8 blocks (the wait for the next chunk is
 // what bounds them), more of them 128 x 32 with chunks of 4. us at 512 / 1024 / 2048 tokens, 1536 x 8960: 53 / 74 / 102
 // (the other form 59 / 77 / 114; 16x16x32 tiles 89 / 110 / 135); 1536 x 1536: 13.7 / 19.1 / 25; 2048 x 1536: 14.0 / 20.0 / 28.
-// 256 to 511 tokens: four K waves per tile, chunks of 8 (333 tokens: 1536 x 8960 35 us, 44 with chunks of 4, 89 for
-// k_mmq<4>, whose sums these are; 1536 x 1536 9.7, 11.5 and 19.8).
+// 256 to 511 tokens, and N % 128 == 64 from 256 on, have four chains over K (k_mmq<4> had them): four K waves per tile,
+// chunks of 8 (333 tokens: 1536 x 8960 35 us, 44 with chunks of 4, 89 for k_mmq<4>; 1536 x 1536 9.7, 11.5 and 19.8).
 template <int EPI>
 static int launch_mmq_narrow(const GemvArgs& a, hipStream_t s) {
-  if (a.T >= 256 && a.T < 512) return launch_mmq_t32<1, 1, 1, 1, 4, 8, EPI>(a, s);
-  if (a.N % 128 || (long)(a.N / 64) * ((a.T + 63) / 64) <= 2 * device_cus()) return launch_mmq_t32<1, 1, 2, 2, 1, 8, EPI>(a, s);
+  if ((a.T >= 256 && a.T < 512) || a.N % 128) return launch_mmq_t32<1, 1, 1, 1, 4, 8, EPI>(a, s);
+  if ((long)(a.N / 64) * ((a.T + 63) / 64) <= 2 * device_cus()) return launch_mmq_t32<1, 1, 2, 2, 1, 8, EPI>(a, s);
   return launch_mmq_t32<1, 1, 4, 1, 1, 4, EPI>(a, s);
 }
 
@@ -536,10 +536,16 @@ static int launch_mmq_narrow(const GemvArgs& a, hipStream_t s) {
 // order is the same whatever the workgroup: 256 x 32, 128 x 64 or 128 x 128, by what the fullest CU costs (us for c
 // workgroups on it, from 17920 x 1536: 256 x 32 20 + 8 (c - 1), 128 x 64 18 + 7.2 (c - 1), 128 x 128 28 + 11 (c - 1)).
 // 17920 x 1536 (us; 16x16x32 tiles before): 77 tokens 20.3 (23.5), 200: 28 (34), 333: 39 (57), 2048: 160 (213).
+// 256 to 511 tokens with fewer than 256 tiles of 128 x 64 keep four chains over K whatever the width (one would double
+// the error: 4608 x 3584 at 300 tokens 1.9e-7 against 1.0e-7; k_mmq<4> 75 us, one wave per tile 42, four 28).
 template <int EPI>
 static int launch_mmq_big(const GemvArgs& a, hipStream_t s) {
-  if constexpr (EPI != EPI_SWIGLU_Q8)
-    if (a.N <= 4096 || a.N % 128) return launch_mmq_narrow<EPI>(a, s);
+  const bool four = a.T >= 256 && a.T < 512 && (long)(a.N / 128) * ((a.T + 63) / 64) < 256;
+  if constexpr (EPI == EPI_SWIGLU_Q8) {
+    if (four) return launch_mmq_t32<2, 1, 1, 1, 4, 8, EPI>(a, s);
+  } else {
+    if (a.N <= 4096 || a.N % 128 || four) return launch_mmq_narrow<EPI>(a, s);
+  }
   const long cu = device_cus();
   const auto full = [&](int rows, int toks) { return (double)(((long)a.N / rows * ((a.T + toks - 1) / toks) + cu - 1) / cu); };
   const double c1 = 10.8 + 7.2 * full(128, 64), c2 = 17 + 11 * full(128, 128), c3 = 12 + 8 * full(256, 32);

@@ -915,10 +915,12 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
 
   // A wave's epilogue takes groups of 4 rows x 32 tokens x 2 lane halves: group q = (token tile, row tile, u) holds rows
   // 8 u + 4 lh .. + 3 of its tile. One K wave: its own RT * TN * 4 groups, from registers. More: all of them leave
-  // their sums in LDS and each adds up its share of the groups in the order of the waves.
-  constexpr int NG = RT * TN * 4 / KW;
+  // their sums in LDS and each adds up its share of the groups in the order of the waves, in f64. SWIGLU_Q8 needs the
+  // 64 rows of a Q8_1 block together: there the first K wave adds up all groups, in fp32 as the epilogue of k_mmq.
+  constexpr bool FIRST = EPI == EPI_SWIGLU_Q8;
+  constexpr int NG = FIRST ? RT * TN * 4 : RT * TN * 4 / KW;
   static_assert(RT * TN * 4 % KW == 0, "whole groups per K wave");
-  typename std::conditional<KW == 1, float, double>::type sum[NG][4];
+  typename std::conditional<KW == 1 || FIRST, float, double>::type sum[NG][4];
   if constexpr (KW > 1) {
     __syncthreads();
     float4* red = (float4*)lds + (size_t)(wr * CW + wc) * (KW * RT * TN * 4 * 64) + lane;
@@ -931,6 +933,7 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
           red[(wk * (RT * TN * 4) + (g * RT + t) * 4 + u) * 64] =
               make_float4(acc[t][g][4 * u], acc[t][g][4 * u + 1], acc[t][g][4 * u + 2], acc[t][g][4 * u + 3]);
     __syncthreads();
+    if (FIRST && wk) return;
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
       for (int e = 0; e < 4; ++e) sum[i][e] = 0;
@@ -952,7 +955,7 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
   if constexpr (EPI == EPI_SWIGLU_Q8) {
     // the wave's 64 rows are one Q8_1 block of 32 outputs per token; lanes l and l ^ 32 hold 16 each: outputs
     // 16 t + 4 u + 2 lh, + 1 in rows 8 u + 4 lh .. of tile t
-    static_assert(EPI != EPI_SWIGLU_Q8 || (RT == 2 && KW == 1), "64 rows per wave");
+    static_assert(EPI != EPI_SWIGLU_Q8 || RT == 2, "64 rows per wave");
 #pragma unroll
     for (int g = 0; g < TN; ++g) {
       const int tok = tokb + 32 * g;

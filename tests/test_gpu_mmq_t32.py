@@ -69,6 +69,42 @@ def test_mmq_t32_store_and_resid(cuda, N, K, T):
     assert (np.abs(got - ref) <= bound + 2.0 ** -48).all()
 
 
+def chains(wb, dw, xq, dx, N, K, T, n):
+    """The sum as n fp32 chains (block b in chain b % n, one rounding a step), joined in float64 in order: [T, N]."""
+    nb = K // 32
+    qw = OQ.q4_0_blocks(wb)[1].reshape(N, K)
+    sq = xq.reshape(T, nb, 32).astype(np.int64).sum(axis=2)
+    acc = np.zeros((n, T, N), np.float32)
+    for b in range(nb):
+        dot = OQ.block_dots(qw[:, 32 * b:32 * b + 32], xq[:, 32 * b:32 * b + 32])[:, :, 0] - 8 * sq[:, b:b + 1]
+        s = dw[:, b].astype(np.float32)[None] * dx[:, b].astype(np.float32)[:, None]         # exact
+        acc[b % n] = (s.astype(np.longdouble) * dot + acc[b % n].astype(np.longdouble)).astype(np.float32)
+    y = np.zeros((T, N))
+    for c in acc:
+        y += c
+    return y
+
+
+# 256 to 511 tokens of fewer than 256 tiles of 128 x 64, and rows an odd multiple of 64 from 256 tokens on
+@pytest.mark.parametrize("N,K,T", [(4224, 384, 256), (4608, 256, 448), (1536, 384, 333), (192, 1280, 513),
+                                   (4160, 384, 520), (64, 256, 1030)])
+def test_sums_of_four_chains(cuda, N, K, T):
+    """These sizes add K as four chains, bit for bit: one chain would double the error of a long K."""
+    import torch
+    wb, dw, xq, dx = problem(N, K, T, N + K + T)
+    W = QM.Q4Mat(wb, N, K, "cuda")
+    xq_d = torch.from_numpy(xq).cuda()
+    xds_d = torch.from_numpy(np.stack([dx, np.zeros_like(dx)], -1)).cuda()
+    want = chains(wb, dw, xq, dx, N, K, T, 4)
+    y = torch.full((T, N), float("nan"), device=cuda)
+    call("q355_mmq_q4_0_q8_1", ptr(W.qs), ptr(W.d), N, K, ptr(xq_d), ptr(xds_d), T, 0, ptr(y), None, None, None, None, None)
+    h = torch.zeros(T, N, dtype=torch.int64, device=cuda)
+    call("q355_mmq_q4_0_q8_1", ptr(W.qs), ptr(W.d), N, K, ptr(xq_d), ptr(xds_d), T, 6, None, ptr(h), None, None, None, None)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(y.cpu().numpy(), want.astype(np.float32))
+    np.testing.assert_array_equal(h.cpu().numpy(), np.rint(want * QM.FIX_SCALE).astype(np.int64))
+
+
 # the tied head of a batch: 16-token tiles up to 16 tokens, 128 x 32 up to 32, 128 x 64 up to 64
 @pytest.mark.parametrize("K,T", [(32, 1), (160, 16), (32, 17), (160, 31), (288, 32), (96, 33), (1536, 63), (128, 64)])
 def test_logits_and_their_partials(cuda, K, T):
@@ -94,7 +130,7 @@ def test_logits_and_their_partials(cuda, K, T):
     assert (np.abs(got - ref) <= bound).all()
 
 
-@pytest.mark.parametrize("T", [512, 577, 1100])
+@pytest.mark.parametrize("T", [256, 300, 448, 512, 577, 1100])
 def test_mmq_t32_swiglu_is_the_quantized_store(cuda, T):
     """SWIGLU_Q8 gives the Q8_1 rule of silu(g) u: codes within one step of those of the STORE sums, and d equal to the
     fp16 of their block maximum / 127 within the error of the hardware exp2 and reciprocal (about 2e-6 relative)."""
