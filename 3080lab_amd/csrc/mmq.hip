@@ -1084,9 +1084,11 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
 
 // RESID_FIX (49 to 255 tokens) and QKV (33 to 255) over a short K (the o and qkv products), where the tiles are few: the K slices of
 // k_mmq_reg's grid (a.mmq_chunk <= 4 blocks each; the block terms of a slice, fp32 or up to 64 tokens exact in f64, added
-// in f64 and rounded to fixed point: the same bytes), but a slice is one wave's 32 x 32 tile, and the workgroup's waves take the slices of one tile and add
-// them through LDS, so an output has one writer: the int64 atomics of the slices (one per output and slice) had been
-// most of the time. A wave loads the blocks of two slices before its first product: one memory latency.
+// in f64 and rounded to fixed point: the same bytes), but a slice is one wave's 32 x 32 tile, and the workgroup's waves
+// take the slices of one tile and add them through LDS, so an output has one writer: the int64 atomics of the slices (one
+// per output and slice) had been most of the time. QKV adds the slices, rounded to the same 2^-48, in f64: the same sums
+// where the fixed point holds them (|sum| < 2^15), and large, infinite and NaN ones stay what they are.
+// A wave loads the blocks of two slices before its first product: one memory latency.
 // Measured (us at 77 / 150 / 250 tokens; k_mmq_reg with atomics before): 1536 x 1536 9.6 / 9.9 / 17.2 (11.8 / 20 / 31), 2048 x
 // 1536 9.8 / 16.5 / 17.7 (16.5 / 24 / 38). Bounded by two memory latencies and the f64 rounding; past one workgroup per
 // CU (registers) by their rounds.
@@ -1094,7 +1096,9 @@ constexpr int S32_KW = 6;
 
 template <int EPI, bool F64>
 __global__ void __launch_bounds__(S32_KW * 64) k_mmq_s32(const GemvArgs a) {
-  __shared__ unsigned long long part[16][64];
+  constexpr bool FIX = EPI == EPI_RESID_FIX;
+  // the f64 rows are padded: a lane reads 12 of them (unpadded 1.5 us more)
+  __shared__ typename std::conditional<FIX, unsigned long long, double>::type part[FIX ? 1 : S32_KW][16][FIX ? 64 : 65];
   const int K = a.K, nb = K / 32, N = a.N, per = a.mmq_chunk;
   const int tid = threadIdx.x, lane = tid & 63, wk = tid >> 6, lc = lane & 31, lh = lane >> 5;
   const int tok0 = blockIdx.z * 32, row0 = blockIdx.x * 32;
@@ -1107,7 +1111,7 @@ __global__ void __launch_bounds__(S32_KW * 64) k_mmq_s32(const GemvArgs a) {
   const unsigned lo = lh ? 0u : 0xFFFFu;                // scales enter as k = 0 of the fp16 product: lanes 0..31
   const v16i zi = {};
   const v16f zf = {};
-  long long sum[16];
+  typename std::conditional<FIX, long long, double>::type sum[16];
 #pragma unroll
   for (int v = 0; v < 16; ++v) sum[v] = 0;
   for (int b0 = wk * per; b0 < nb; b0 += 2 * S32_KW * per) {          // two of this wave's slices at a time
@@ -1144,21 +1148,29 @@ __global__ void __launch_bounds__(S32_KW * 64) k_mmq_s32(const GemvArgs a) {
           }
         }
 #pragma unroll
-      for (int v = 0; v < 16; ++v) sum[v] += to_fix(s[v]);
+      for (int v = 0; v < 16; ++v) {
+        if constexpr (FIX) sum[v] += to_fix(s[v]);
+        else sum[v] += rint(s[v] * FIX_SCALE) * FIX_INV;
+      }
     }
   }
-  for (int e = tid; e < 16 * 64; e += S32_KW * 64) part[e >> 6][e & 63] = 0;
-  __syncthreads();
+  if constexpr (FIX) {
+    for (int e = tid; e < 16 * 64; e += S32_KW * 64) part[0][e >> 6][e & 63] = 0;
+    __syncthreads();
 #pragma unroll
-  for (int v = 0; v < 16; ++v) atomicAdd(&part[v][lane], (unsigned long long)sum[v]);      // integers: any order
+    for (int v = 0; v < 16; ++v) atomicAdd(&part[0][v][lane], (unsigned long long)sum[v]);      // integers: any order
+  } else {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) part[wk][v][lane] = sum[v];
+  }
   __syncthreads();
   for (int e = tid; e < 512; e += S32_KW * 64) {                      // 2 consecutive rows of one token
     const int r = (e & 15) * 2, t = e >> 4;
     const int pv = 4 * (r >> 3) + (r & 3), pl = t + 32 * ((r >> 2) & 1);
     const int tk = tok0 + t, row = row0 + r;
     if (tk >= a.T) continue;
-    const long long f0 = (long long)part[pv][pl], f1 = (long long)part[pv + 1][pl];
-    if constexpr (EPI == EPI_RESID_FIX) {
+    if constexpr (FIX) {
+      const long long f0 = (long long)part[0][pv][pl], f1 = (long long)part[0][pv + 1][pl];
       longlong2* y = (longlong2*)(a.yfix + (size_t)tk * N + row);
       longlong2 h = *y;
       h.x += f0;
@@ -1167,7 +1179,14 @@ __global__ void __launch_bounds__(S32_KW * 64) k_mmq_s32(const GemvArgs a) {
     } else {                                                          // as k_qkv_finish: the two rows are a RoPE pair
       const int nq = a.nh * HD, nk = a.nkv * HD, pos = a.pos[tk];
       const int pg = a.block_table[(size_t)(tk * a.seq_stride) * a.bt_stride + pos / PAGE];
-      const double v0 = from_fix(f0) + (double)a.aux[row], v1 = from_fix(f1) + (double)a.aux[row + 1];
+      double v0 = 0.0, v1 = 0.0;
+#pragma unroll
+      for (int w = 0; w < S32_KW; ++w) {
+        v0 += part[w][pv][pl];
+        v1 += part[w][pv + 1][pl];
+      }
+      v0 += (double)a.aux[row];
+      v1 += (double)a.aux[row + 1];
       if (row < nq + nk) {
         const int i = (row % HD) >> 1;
         const double c = a.rope_cos[(size_t)pos * (HD / 2) + i], s = a.rope_sin[(size_t)pos * (HD / 2) + i];

@@ -40,3 +40,37 @@ def test_prefill_qkv_sums_as_the_split_product(cuda, H, NH, NKV, P):
     torch.cuda.synchronize()
     assert int((vc != 0).sum()) > P * NKV * 100
     assert torch.equal(kc, dec.kc[0]) and torch.equal(vc, dec.vc[0])
+
+
+@pytest.mark.parametrize("T", [20, 40, 100, 300])
+def test_fused_qkv_keeps_large_and_non_finite_values(cuda, T):
+    """Products past the residual stream's fixed point (2^15), past fp16, infinite and NaN come out of the fused call of
+    every form as the float64 sum rounded to fp16."""
+    import torch
+    nh, nkv, K = 4, 1, 512
+    N, nb = (nh + 2 * nkv) * 128, K // 32
+    rng = np.random.default_rng(T)
+    qs = np.full((N, nb, 16), 0x99, np.uint8)                             # every weight d (9 - 8)
+    d = np.full((N, nb), 0.25, np.float16)
+    row = {"large": (nh + nkv) * 128, "over": (nh + nkv) * 128 + 1, "inf": (nh + nkv) * 128 + 2, "nan": (nh + nkv) * 128 + 37}
+    d[row["large"]], d[row["over"]] = 0.9, 20000
+    d[row["inf"], nb // 2], d[row["nan"], nb - 1] = np.inf, np.nan
+    W = QM.Q4Mat(np.concatenate([d.view(np.uint8).reshape(N, nb, 2), qs], 2).reshape(-1, 18), N, K, "cuda")
+    xq = np.full((T, K), 100, np.int8) - rng.integers(0, 3, (T, K)).astype(np.int8)
+    xds = np.ones((T, nb, 2), np.float16)
+    with np.errstate(invalid="ignore", over="ignore"):
+        dots = xq.reshape(T, nb, 32).astype(np.float64).sum(2)
+        want = (dots[:, None] * d.astype(np.float64)[None]).sum(2).astype(np.float16)[:, (nh + nkv) * 128:]
+    assert 2 ** 15 < want[0, 0] < 65504 and want[0, 1] == np.inf and want[0, 2] == np.inf and np.isnan(want[0, 37])
+    t = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    pages = (T + 63) // 64
+    kc = torch.zeros(pages, nkv, 64, 128, dtype=torch.float16, device=cuda)
+    vc, q = torch.zeros_like(kc), torch.zeros(T, nh * 128, dtype=torch.float16, device=cuda)
+    args = [t(xq), t(xds), t(np.zeros(N, np.float32)), t(np.ones((512, 64), np.float32)), t(np.zeros((512, 64), np.float32)),
+            t(np.arange(T, dtype=np.int32)), t(np.arange(pages, dtype=np.int32))]
+    p = [ptr(a) for a in args]
+    call("q355_mmq_qkv_rope", ptr(W.qs), ptr(W.d), N, K, p[0], p[1], T, *p[2:], pages, 0, ptr(kc), ptr(vc), ptr(q), None, nh,
+         nkv)
+    torch.cuda.synchronize()
+    got = vc.reshape(-1, 128)[:T].cpu().numpy()
+    np.testing.assert_array_equal(got, want)
