@@ -16,7 +16,7 @@
 // four tokens: per sub-block two MFMAs of 8 weights a lane. One fp32 chain per block index mod 4, added at the end.
 // More tokens would repeat those MFMAs per four of them, so there a 4 x 4 transpose of the lane groups (eight lane
 // swaps) spreads each block over its k-groups, and a block against 16 tokens is two MFMAs, the weights of the other
-// sub-block zeroed.
+// sub-block zeroed. It keeps the same four chains, so that a sequence's logits have the same bits whatever the batch.
 // Either way a sub-block is an exact int32 sum of (v - 32) q_x, and sc0 C0 + sc1 C1 (exact int32, |.| < 2^24) is scaled by
 // d d_x (exact fp32 product) into fp32 accumulators.
 //
@@ -84,10 +84,11 @@ __device__ __forceinline__ void transpose4(unsigned (&w)[4]) {
   swap16(w[2], w[3]);
 }
 
-// Four blocks against TG groups of 16 tokens: xl = this lane's token and k-group, xd = its accumulators' tokens
+// Four blocks against TG groups of 16 tokens: xl = this lane's token and k-group, xd = its accumulators' tokens; block u
+// adds to the chain acc[u]
 template <int TG>
 __device__ __forceinline__ void q6m_group_t(const Q6Group& G, const int8_t* xl, int xstride, const float* xd, bool sub0,
-                                            float (&acc)[TG][4]) {
+                                            float (&acc)[4][TG][4]) {
   constexpr int TT = 16 * TG;
   long w[4];
   q6m_weights(G, w);
@@ -115,7 +116,7 @@ __device__ __forceinline__ void q6m_group_t(const Q6Group& G, const int8_t* xl, 
       const float s[4] = {G.d * dx.x, G.d * dx.y, G.d * dx.z, G.d * dx.w};
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        acc[g][v] = fmaf(s[v], (float)(__mul24(sc0, c0[v]) + __mul24(sc1, c1[v])), acc[g][v]);
+        acc[u][g][v] = fmaf(s[v], (float)(__mul24(sc0, c0[v]) + __mul24(sc1, c1[v])), acc[u][g][v]);
     }
   }
 }
@@ -177,16 +178,19 @@ __global__ void __launch_bounds__(NW * 64) k_mmq_q6k_logits(const GemvArgs a) {
   const int8_t* xl = OWN ? xs + (size_t)(li & 3) * xstride + (own ? 32 * lg : K) : xs + (size_t)li * xstride + 8 * lg;
   const int step = !OWN || own ? 128 : 0;
   const float* xdl = OWN ? xd + lg * TT : xd + 4 * lg;
-  float acc[TQ][4];
+  constexpr int NC = OWN ? 1 : 4;                                  // chains in this lane's registers
+  float acc[NC][TQ][4];
 #pragma unroll
-  for (int q = 0; q < TQ; ++q)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) acc[q][v] = 0.f;
+    for (int q = 0; q < TQ; ++q)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[c][q][v] = 0.f;
   for (int g = 0; g < ng; g += AHEAD)
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i)
       if (g + i < ng) {                                             // uniform
-        if constexpr (OWN) q6m_group<TQ>(G[i], xl, xstride, xdl, acc);
+        if constexpr (OWN) q6m_group<TQ>(G[i], xl, xstride, xdl, acc[0]);
         else q6m_group_t<TG>(G[i], xl, xstride, xdl, lg < 2, acc);
         if (g + i + AHEAD < ng) q6m_load(G[i], a, tile, g + i + AHEAD, nb, lane);
         xl += step;
@@ -208,11 +212,12 @@ __global__ void __launch_bounds__(NW * 64) k_mmq_q6k_logits(const GemvArgs a) {
     if constexpr (OWN) {                                            // the sum of the four chains; lane group lg takes token lg
       float s[4];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) s[v] = xsum32(xsum16(acc[q][v]));
+      for (int v = 0; v < 4; ++v) s[v] = xsum32(xsum16(acc[0][q][v]));
       finish(4 * q + lg, lg == 0 ? s[0] : lg == 1 ? s[1] : lg == 2 ? s[2] : s[3]);
     } else {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) finish(16 * q + 4 * lg + v, acc[q][v]);
+      for (int v = 0; v < 4; ++v)
+        finish(16 * q + 4 * lg + v, (acc[0][q][v] + acc[1][q][v]) + (acc[2][q][v] + acc[3][q][v]));
     }
   }
   __syncthreads();

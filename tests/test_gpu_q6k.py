@@ -123,6 +123,31 @@ def test_mmq_q6k_logits_forms(cuda, N, K, T):
     assert np.array_equal(pidx.cpu().numpy(), parts.argmax(axis=2) + 64 * np.arange(N // 64)[None])
 
 
+@pytest.mark.parametrize("N,K", [(192, 256), (256, 1536), (1024, 768)])
+def test_mmq_q6k_logits_do_not_depend_on_the_batch(cuda, N, K):
+    """A token's logits have the same bits alone, in a batch of up to 8, 16 or 32 tokens, and at any place in it."""
+    import torch
+    rng = np.random.default_rng(N + K)
+    b = random_q6_k(N * K // 256, rng, d=0.0005)
+    W = QM.Q6KMat(b, N, K, "cuda")
+    q, d, s = OQ.quantize_q8_1(rng.standard_normal((32, K), dtype=np.float32))
+    xq = torch.from_numpy(q).cuda()
+    xds = torch.from_numpy(np.stack([d, s], -1)).cuda()
+
+    def logits(lo, hi):
+        T = hi - lo
+        y = torch.full((T, N), float("nan"), device=cuda)
+        pmax = torch.zeros(T, N // 64, device=cuda)
+        pidx = torch.zeros(T, N // 64, dtype=torch.int32, device=cuda)
+        call("q355_mmq_q6k_logits", ptr(W.lo), ptr(W.hi), ptr(W.sc), ptr(W.d), N, K, ptr(xq[lo:]), ptr(xds[lo:]), T, ptr(y),
+             ptr(pmax), ptr(pidx))
+        return y
+
+    full = logits(0, 32)
+    for lo, hi in ((0, 1), (0, 8), (24, 32), (0, 9), (5, 21), (15, 32), (31, 32)):
+        assert torch.equal(logits(lo, hi), full[lo:hi]), (lo, hi)
+
+
 @pytest.mark.parametrize("B", [8, 32])
 def test_batched_decode_with_q6k_head(cuda, B):
     """BatchedDecoder with llama.cpp's Q6_K output.weight (int8 MMQ layers, Q6_K MFMA head), teacher-forced
