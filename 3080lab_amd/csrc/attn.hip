@@ -440,9 +440,10 @@ __device__ __forceinline__ void attn_merge_head(const double* __restrict__ P, in
   const int lane = threadIdx.x & 63;
   const double* pc = P + (size_t)min(lane, maxc - 1) * (HD + 2);
   const double mc = pc[HD], lc = pc[HD + 1];
-  // the first 8 chunks do not wait for the position (nch); the rest of up to 32 follows in one go, so a context of 2048
-  // positions costs two memory latencies (at position 1811, four of 8 chunks each: the 8-layer step 253 us against 249)
-  constexpr int NV = 32;
+  // The first 8 chunks do not wait for the position (nch); the others follow 16 at a time, one memory latency each. us of
+  // the O product (graph, 1536 x 1536) in groups of 8 / 16 / 32 chunks, 1 token at position 140: 3.9 / 3.9 / 4.15, at 1811:
+  // 5.6 / 5.2 / 5.4; 4 tokens 8.9 / 8.9 / 10.1 and 15.5 / 14.3 / 15.0 (32 hold 128 VGPRs, which every context pays for).
+  constexpr int NV = 16;
   double2 v[NV];
 #pragma unroll
   for (int u = 0; u < 8; ++u) v[u] = ((const double2*)(P + (size_t)min(u, maxc - 1) * (HD + 2)))[lane];
