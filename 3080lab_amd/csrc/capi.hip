@@ -628,11 +628,29 @@ static int mmq_slices(int N, int K) {
   return KS < 1 || most < 1 ? 1 : KS < most ? KS : most;
 }
 
-// 49 (QKV: 33) to 255 tokens: slices of up to four blocks run in k_mmq_s32 (1536 x 1536 at 64 tokens 9.4 us against 12.3, at
-// 40 tokens 9.2 against 8.6). Longer ones (the down product) stay on the 16-token
-// kernels: a wave would run its 18 blocks one latency after another (1536 x 8960, 77 / 200 tokens: 25.5 / 48 us against
-// 23.5 / 41).
+// Where k_mmq_s32 adds the slices of up to 255 tokens: slices of up to four blocks (longer ones, as the down product's, stay
+// on the 16-token kernels: a wave would run its 18 blocks one latency after another; 1536 x 8960, 77 / 200 tokens: 25.5 / 48
+// us against 23.5 / 41). It takes 1.2 us and, for each round of one workgroup per CU, 3.2 + 0.36 a slice, whatever the tokens
+// of a tile; the 16-token kernels pay for each output and slice (an int64 atomic): 4 us + 5.5 a million (7 up to 64 tokens,
+// whose terms are f64), and no less than 8. RESID_FIX takes it from 49 tokens where that is the less, by more than the fits
+// are off (8 %). us of the two: 1536 x 1536 (12 slices) 49 / 128 tokens 8.8 / 9.4 against 11.1 / 17.6, 768 x 1536 96 / 128
+// tokens 9.3 / 9.4 against 8.7 / 10.0, 192 x 8960 (70) 64 / 255 tokens 28 / 30 against 9.7 / 24, 6144 x 256 (2) 64 / 255
+// tokens 9.0 / 24 against 8.0 / 21.
+// QKV, whose other form is one fp32 chain over K (2048 x 1536 21 us), takes it for up to two rounds (2560 x 768 at 192 / 224
+// tokens 13.4 / 17.5 us against 13.9).
 static bool mmq_short_slices(int K, int KS) { return (K / 32 + KS - 1) / KS <= 4; }
+static bool mmq_resid_s32(const GemvArgs& a, int KS) {
+  if (a.T <= 48 || !mmq_short_slices(a.K, KS)) return false;
+  const long wg = (long)(a.N / 32) * ((a.T + 31) / 32), cu = device_cus();
+  const double s32 = 1.2 + (double)((wg + cu - 1) / cu) * (3.2 + 0.36 * KS);
+  const double t16 = 4 + (a.T <= 64 ? 7e-6 : 5.5e-6) * a.N * KS * a.T;
+  return 1.08 * s32 < (t16 > 8 ? t16 : 8);
+}
+static int mmq_qkv_s32_max_t(int N, int K) {
+  if (!mmq_short_slices(K, mmq_slices(N, K))) return 0;
+  const long t = 2L * device_cus() * 32 / N * 32;
+  return t < 255 ? (int)t : 255;
+}
 template <int EPI>
 static int launch_mmq_s32(const GemvArgs& a, int KS, hipStream_t s) {
   GemvArgs b = a;
@@ -658,7 +676,7 @@ static int launch_mmq_tg(const GemvArgs& a, int KS, hipStream_t s) {
     if ((a.N % 128 == 0 && (a.N / 128) * ((a.T + 63) / 64) >= 256) || (a.T >= 256 && (EPI != EPI_SWIGLU_Q8 || a.N % 128 == 0)))
       return launch_mmq_big<EPI>(a, s);
   if constexpr (EPI == EPI_RESID_FIX)
-    if (a.T > 48 && mmq_short_slices(a.K, KS)) return launch_mmq_s32<EPI>(a, KS, s);
+    if (mmq_resid_s32(a, KS)) return launch_mmq_s32<EPI>(a, KS, s);
   // up to 64 tokens (decode batches): 16-token workgroups, several per CU, hide each other's latencies; what is left of
   // the larger calls: 32- or 64-token workgroups reuse every staged weight block 2 or 4 times
   if (a.T <= 64) return launch_mmq<1, EPI>(a, KS, s);
@@ -1060,7 +1078,8 @@ extern "C" int q355_qkv_finish(int64_t* acc, const float* bias, const float* rop
 // below 256 tokens it is one fp32 chain over the whole K (k_mmq_t32), where the split form adds f64 or short slices.
 extern "C" int q355_mmq_qkv_fused_max_t(int N, int K) {
   if (N < 64 || N % 64 || K < 32 || K % 32) return 0;
-  return mmq_short_slices(K, mmq_slices(N, K)) ? 255 : mmq_qkv_in_registers(N, K) ? 32 : 0;
+  const int t = mmq_qkv_s32_max_t(N, K);
+  return t < 32 && mmq_qkv_in_registers(N, K) ? 32 : t;
 }
 
 // QKV product with the finish fused into its epilogue: every output has one writer (no K split), so no int64
@@ -1089,8 +1108,7 @@ extern "C" int q355_mmq_qkv_rope(const uint8_t* qs, const void* d, int N, int K,
                           : launch_mmq_r_tg<2, EPI_QKV, false>(a, (hipStream_t)stream);
     if (r >= 0) return r;
   }
-  const int KS = mmq_slices(N, K);
-  if (T < 256 && mmq_short_slices(K, KS)) return launch_mmq_s32<EPI_QKV>(a, KS, (hipStream_t)stream);
+  if (T <= mmq_qkv_s32_max_t(N, K)) return launch_mmq_s32<EPI_QKV>(a, mmq_slices(N, K), (hipStream_t)stream);
   return launch_mmq_big<EPI_QKV>(a, (hipStream_t)stream);
 }
 

@@ -174,3 +174,13 @@ def test_weights_from_gguf_roundtrip(tmp_path):
     for a, b in zip(w["layers"], w2["layers"]):
         for k in a:
             assert np.array_equal(np.asarray(a[k]).reshape(-1), np.asarray(b[k]).reshape(-1)), k
+
+
+@pytest.mark.parametrize("N,K,t", [(2048, 1536, 255),                      # Qwen2.5-1.5B
+                                   (2560, 2048, 0), (4608, 3584, 0),       # slices past four blocks, K past the registers
+                                   (1536, 960, 32), (768, 1088, 32),       # K % 128 != 0: slices of five blocks
+                                   (2560, 768, 192), (4608, 512, 96),      # two rounds of workgroups
+                                   (512, 2048, 255), (768, 896, 255), (2048, 100, 0), (100, 1536, 0)])
+def test_qkv_fused_max_t(N, K, t):
+    """Up to how many tokens (below 256) the fused QKV sums as the split product does, for 256 compute units."""
+    assert hip.call("q355_mmq_qkv_fused_max_t", N, K) == t
