@@ -554,14 +554,18 @@ static int launch_mmq_big(const GemvArgs& a, hipStream_t s) {
   return launch_mmq_t32<2, 1, 2, 2, 1, 4, EPI>(a, s);
 }
 
-// LOGITS over a large vocabulary (N % 128 == 0) for up to 64 tokens: the LDS-tiled kernels with 128 rows and all tokens
-// in one workgroup, so each weight is read once. Up to 16 tokens k_mmq_tile (16-token MFMAs: no work for padding), above
+// LOGITS over a large vocabulary (N % 128 == 0) for up to 64 tokens: the LDS-tiled kernels with all tokens in one
+// workgroup, so each weight is read once. Up to 16 tokens k_mmq_tile (128 rows; 16-token MFMAs: no work for padding), above
 // that k_mmq_t32, whose fp32 sums are the same bits (151936 x 1536, us at 16 / 24 / 32 / 48 / 64 tokens: k_mmq_tile 31 / 43 /
-// 43 / 66 / 67, k_mmq_t32 36 / 36 / 36 / 53 / 54; chunks of 8 blocks 58 at 32 tokens and 66 at 64: half the workgroups per
-// CU; two K waves per tile 34 and 61).
+// 43 / 66 / 67, k_mmq_t32 of 128 rows 36 / 36 / 36 / 53 / 54; chunks of 8 blocks 58 at 32 tokens and 66 at 64: half the
+// workgroups per CU; two K waves per tile 34 and 61). Up to 32 tokens a vocabulary of up to two such workgroups per CU
+// leaves room for chunks of 8, in 64-row workgroups of one wave (32768 x 2048 24 us, 128 rows 28, k_mmq_tile 23; 65536 x 1536
+// 22, 25 and 23; 73728 x 1536 36, 26 and 27).
 static int launch_mmq_logits_tile(const GemvArgs& a, hipStream_t s) {
   if (a.T > 32) return launch_mmq_t32<2, 1, 2, 2, 1, 4, EPI_LOGITS>(a, s);
-  if (a.T > 16) return launch_mmq_t32<2, 1, 2, 1, 1, 4, EPI_LOGITS>(a, s);
+  if (a.T > 16)
+    return a.N / 128 <= 2 * device_cus() ? launch_mmq_t32<2, 1, 1, 1, 1, 8, EPI_LOGITS>(a, s)
+                                         : launch_mmq_t32<2, 1, 2, 1, 1, 4, EPI_LOGITS>(a, s);
   constexpr size_t lds = 2 * LdsTile<2, TILE_CB>::BUF;
   hipLaunchKernelGGL(k_mmq_tile<2>, dim3(a.N / 128, 1, 1), dim3(128), lds, s, a);
   return launched("mmq");

@@ -105,12 +105,13 @@ def test_sums_of_four_chains(cuda, N, K, T):
     np.testing.assert_array_equal(h.cpu().numpy(), np.rint(want * QM.FIX_SCALE).astype(np.int64))
 
 
-# the tied head of a batch: 16-token tiles up to 16 tokens, 128 x 32 up to 32, 128 x 64 up to 64
-@pytest.mark.parametrize("K,T", [(32, 1), (160, 16), (32, 17), (160, 31), (288, 32), (96, 33), (1536, 63), (128, 64)])
-def test_logits_and_their_partials(cuda, K, T):
+# the tied head of a batch: 16-token tiles up to 16 tokens, 64 x 32 (up to 65536 rows) or 128 x 32 up to 32, 128 x 64 up to 64
+@pytest.mark.parametrize("N,K,T", [(32896, 32, 1), (32896, 160, 16), (32896, 32, 17), (32896, 160, 31), (32896, 288, 32),
+                                   (65536, 544, 32), (65664, 32, 17), (65664, 160, 31), (65664, 288, 32), (32896, 96, 33),
+                                   (32896, 1536, 63), (32896, 128, 64)])
+def test_logits_and_their_partials(cuda, N, K, T):
     """Logits within the bound; every (max, lowest row) over 64 rows is that of the stored logits, also without them."""
     import torch
-    N = 128 * 256 + 128
     wb, dw, xq, dx = problem(N, K, T, K + T)
     W = QM.Q4Mat(wb, N, K, "cuda")
     xq_d = torch.from_numpy(xq).cuda()
