@@ -536,16 +536,21 @@ static int launch_mmq_narrow(const GemvArgs& a, hipStream_t s) {
 // order is the same whatever the workgroup: 256 x 32, 128 x 64 or 128 x 128, by what the fullest CU costs (us for c
 // workgroups on it, from 17920 x 1536: 256 x 32 20 + 8 (c - 1), 128 x 64 18 + 7.2 (c - 1), 128 x 128 28 + 11 (c - 1)).
 // 17920 x 1536 (us; 16x16x32 tiles before): 77 tokens 20.3 (23.5), 200: 28 (34), 333: 39 (57), 2048: 160 (213).
-// 256 to 511 tokens with fewer than 256 tiles of 128 x 64 keep four chains over K whatever the width (one would double
-// the error: 4608 x 3584 at 300 tokens 1.9e-7 against 1.0e-7; k_mmq<4> 75 us, one wave per tile 42, four 28).
+// Fewer than 256 tiles of 128 x 64 below 512 tokens: the narrow forms, whatever the width. From 256 tokens these keep four
+// chains over K (one would double the error: 4608 x 3584 at 300 tokens 1.9e-7 against 1.0e-7; k_mmq<4> 75 us, one wave per
+// tile 42, four 28); the fused QKV of fewer tokens waits less in their chunks of 8 (4608 x 3584 at 77 tokens 25 us against 43,
+// 16x16x32 tiles 40).
+// RESID_FIX reads and writes 8 bytes an output: with one row tile per wave (128 x 32) more waves share that, 4224 x 1536 at
+// 512 tokens 25.5 us against 33.4, 17920 x 1536 at 1024 128 against 145 (16x16x32 tiles 29.3 and 130).
 template <int EPI>
 static int launch_mmq_big(const GemvArgs& a, hipStream_t s) {
-  const bool four = a.T >= 256 && a.T < 512 && (long)(a.N / 128) * ((a.T + 63) / 64) < 256;
+  const bool few = a.T < 512 && (long)(a.N / 128) * ((a.T + 63) / 64) < 256;
   if constexpr (EPI == EPI_SWIGLU_Q8) {
-    if (four) return launch_mmq_t32<2, 1, 1, 1, 4, 8, EPI>(a, s);
+    if (few) return launch_mmq_t32<2, 1, 1, 1, 4, 8, EPI>(a, s);
   } else {
-    if (a.N <= 4096 || a.N % 128 || four) return launch_mmq_narrow<EPI>(a, s);
+    if (a.N <= 4096 || a.N % 128 || few) return launch_mmq_narrow<EPI>(a, s);
   }
+  if constexpr (EPI == EPI_RESID_FIX) return launch_mmq_t32<1, 1, 4, 1, 1, 4, EPI>(a, s);
   const long cu = device_cus();
   const auto full = [&](int rows, int toks) { return (double)(((long)a.N / rows * ((a.T + toks - 1) / toks) + cu - 1) / cu); };
   const double c1 = 10.8 + 7.2 * full(128, 64), c2 = 17 + 11 * full(128, 128), c3 = 12 + 8 * full(256, 32);
