@@ -528,7 +528,9 @@ static int launch_mmq_t32(const GemvArgs& a, hipStream_t s) {
 template <int EPI>
 static int launch_mmq_narrow(const GemvArgs& a, hipStream_t s) {
   if ((a.T >= 256 && a.T < 512) || a.N % 128) return launch_mmq_t32<1, 1, 1, 1, 4, 8, EPI>(a, s);
-  if ((long)(a.N / 64) * ((a.T + 63) / 64) <= 2 * device_cus()) return launch_mmq_t32<1, 1, 2, 2, 1, 8, EPI>(a, s);
+  // past 65535 groups of 32 tokens (grid.z) the 64-token form as well
+  if ((long)(a.N / 64) * ((a.T + 63) / 64) <= 2 * device_cus() || a.T > 65535 * 32)
+    return launch_mmq_t32<1, 1, 2, 2, 1, 8, EPI>(a, s);
   return launch_mmq_t32<1, 1, 4, 1, 1, 4, EPI>(a, s);
 }
 

@@ -74,3 +74,31 @@ def test_fused_qkv_keeps_large_and_non_finite_values(cuda, T):
     torch.cuda.synchronize()
     got = vc.reshape(-1, 128)[:T].cpu().numpy()
     np.testing.assert_array_equal(got, want)
+
+
+def test_fused_qkv_of_more_than_65535_tiles_of_32_tokens(cuda):
+    """The call takes up to 65535 x 64 tokens, the grid's third dimension 65535 workgroups: past 65535 x 32 tokens the
+    workgroups hold 64 tokens, and the last tokens come out as a short call gives them."""
+    import torch
+    nh, nkv, K, T = 4, 1, 32, 65535 * 32 + 33
+    N = (nh + 2 * nkv) * 128
+    rng = np.random.default_rng(3)
+    d = np.full((N, 1), 0.01, np.float16)
+    qs = rng.integers(0, 256, (N, 1, 16), dtype=np.uint8)
+    W = QM.Q4Mat(np.concatenate([d.view(np.uint8).reshape(N, 1, 2), qs], 2).reshape(-1, 18), N, K, "cuda")
+    xq = torch.randint(-127, 128, (T, K), device=cuda, dtype=torch.int32, generator=torch.Generator(cuda).manual_seed(1)).to(torch.int8)
+    xds = torch.full((T, 1, 2), 0.01, dtype=torch.float16, device=cuda)
+    bias = torch.zeros(N, device=cuda)
+    cos, sin = torch.ones(64, 64, device=cuda), torch.zeros(64, 64, device=cuda)
+    pos = torch.zeros(T, dtype=torch.int32, device=cuda)
+    table = torch.zeros(1, dtype=torch.int32, device=cuda)
+    kc, vc = (torch.zeros(1, nkv, 64, 128, dtype=torch.float16, device=cuda) for _ in range(2))
+
+    def run(first, n):
+        q = torch.zeros(n, nh * 128, dtype=torch.float16, device=cuda)
+        call("q355_mmq_qkv_rope", ptr(W.qs), ptr(W.d), N, K, ptr(xq[first:]), ptr(xds[first:]), n, ptr(bias), ptr(cos), ptr(sin),
+             ptr(pos), ptr(table), 1, 0, ptr(kc), ptr(vc), ptr(q), None, nh, nkv)
+        return q
+
+    q = run(0, T)
+    assert torch.equal(q[-100:], run(T - 100, 100)) and torch.equal(q[:600], run(0, 600)) and bool((q[-100:] != 0).any())
