@@ -166,9 +166,12 @@ int q355_attn_o_resid(const uint8_t* qs, const void* d, int N, const double* par
 int q355_rmsnorm_fix_q8_1(const int64_t* h, const float* w, int8_t* xq, void* xds, int T, int H, double eps,
                           void* stream);
 
-/* Q4_0 x Q8_1 product of T tokens on v_mfma_i32_16x16x32_i8 (exact int32 block dots), N % 64 == 0.
+/* Q4_0 x Q8_1 product of T tokens on int8 MFMA (exact int32 block dots; 16x16x32 tiles for decode batches and short
+ * prompts, 32x32x32 ones otherwise), N % 64 == 0.
  * epi 0: y fp32 [T][N] = W x;  5: argmax partials pmax/pidx [T][q355_mmq_nparts(N)] and, if y is given, logits y [T][N];
- * 6: yfix [T][N] += W x (int64 fixed point, K-sliced, integer atomics);
+ * 6: yfix [T][N] += W x (int64 fixed point). The call needs yfix for itself while it runs: decode batches add K slices with
+ *    integer atomics, but from 49 tokens or 32768 rows on, depending on N, K and T, each output is read, added to and
+ *    written by one lane, so what another launch (on another stream) adds to the same yfix meanwhile can be lost;
  * 4: rows interleaved (gate, up): y fp32 [T][N/2] = silu(g) * u;
  * 7: rows interleaved (gate, up): Q8_1 of silu(g) * u into oq [T][N/2], ods [T][N/64].
  * Replaces gemm_q4i8_source / gemm_q4i8_ms_source with epilogues resid / swiglu_q8
@@ -264,9 +267,9 @@ int q355_qkv_finish(int64_t* acc, const float* bias, const float* rope_cos, cons
                     const int32_t* pos, const int32_t* block_table, int bt_stride, int seq_stride, void* kcache,
                     void* vcache, void* qout, int nh, int nkv, int T, void* stream);
 
-/* QKV: Q4_0 x Q8_1 product of T tokens on int8 MFMA (register-resident for T <= 32 and K <= 1536, LDS-tiled
- * otherwise) with the QKV finish in its epilogue: + bias, RoPE, fp16 q out [T][nh*128], fp16 K/V cache rows at pos[j] of sequence j * seq_stride
- * (arguments as q355_qkv_finish). q64 (optional, may be NULL): the same fp16 q values widened to f64 [T][nh*128],
+/* QKV: Q4_0 x Q8_1 product of T tokens on int8 MFMA (register-resident for T <= 32 and K <= 1536, K slices added in LDS
+ * up to 255 tokens where they are short, LDS-tiled otherwise) with the QKV finish in its epilogue: + bias, RoPE, fp16 q out
+ * [T][nh*128], fp16 K/V cache rows at pos[j] of sequence j * seq_stride (arguments as q355_qkv_finish). q64 (optional, may be NULL): the same fp16 q values widened to f64 [T][nh*128],
  * the input of q355_attn_decode_f64. N = (nh + 2 nkv) * 128 in the device row order, N % 128 == 0.
  * Replaces gemm_q4i8_ms_source with the 'biasf_kv' epilogue (lab/qwen_batched.py:1271-1561, 1316-1362). */
 int q355_mmq_qkv_rope(const uint8_t* qs, const void* d, int N, int K, const int8_t* xq, const void* xds, int T,
