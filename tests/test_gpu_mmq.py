@@ -282,8 +282,8 @@ def test_batched_equals_single_sequence(small):
     check_greedy(got[0], ref, margins, "batched vs batch-1")
 
 
-# Prefill-size products (the LDS-tiled kernel: N % 128 == 0 and at least 256 tiles of 128 x 64): the full
-# product is too large for the oracle, so a random subset of rows is checked against it.
+# Prefill-size products (k_mmq_t32; N % 128 == 0 and at least 256 tiles of 128 x 64): the full product is too large for the
+# oracle, so a random subset of rows is checked against it.
 @pytest.mark.parametrize("N,K,T", [(17920, 1536, 300), (4096, 1536, 2100), (4096, 1568, 700)])
 def test_mmq_tile_store(cuda, N, K, T):
     import torch

@@ -1,4 +1,4 @@
-"""The prefill products on 32 x 32 x 32 int8 tiles (k_mmq_t32) at the sizes where they can go wrong: K shorter than a
+"""The prefill products on 32 x 32 x 32 int8 tiles (k_mmq_t32, k_mmq_s32) at the sizes where they can go wrong: K shorter than a
 staged chunk of 4 or 8 blocks, K that ends inside one, token counts around a tile, every tile form, activations of -128
 and subnormal scales.
 
@@ -41,16 +41,19 @@ def reference(wb, dw, xq, dx, N, K, T):
     return y, (nb + 1) * 2.0 ** -23 * mag
 
 
-# dispatch: 49 to 255 tokens over a short K: RESID_FIX slices of one tile per workgroup (k_mmq_s32, f64 up to 64 tokens),
-# STORE from 65 tokens eight K waves; then up to 4096 rows one 32 x 32 tile per wave, with four K waves from 256 to 511
-# tokens (64 x 64 workgroups from 512, 128 x 32 past two per CU); wider 256 x 32, 128 x 64 or 128 x 128
+# dispatch: 49 to 255 tokens over a short K: RESID_FIX slices of one tile per workgroup (k_mmq_s32, f64 up to 64 tokens; one
+# to three slices a wave), STORE from 65 tokens eight K waves; then up to 4096 rows one 32 x 32 tile per wave, with four K
+# waves from 256 to 511 tokens (64 x 64 workgroups from 512, 128 x 32 past two per CU), the residual at every width; wider
+# STORE 256 x 32 (77 and 200 tokens of 17920 rows), 128 x 64 or 128 x 128 (333 and 1100)
 @pytest.mark.parametrize("N,K,T", [(64, 32, 49), (128, 224, 64), (1536, 1536, 50), (64, 32, 65), (128, 288, 97),
+                                   (1536, 1536, 97), (1024, 2048, 100), (512, 4096, 250), (2048, 128, 255),
                                    (1536, 160, 200), (192, 8960, 70), (4096, 96, 255),
                                    (64, 32, 256), (128, 288, 257), (1536, 160, 333), (192, 96, 511), (4096, 64, 300),
                                    (128, 32, 512), (64, 96, 545), (192, 128, 513), (128, 160, 575),
                                    (128, 288, 576), (4096, 96, 513), (2048, 32, 1100), (4096, 288, 700),
                                    (4224, 32, 512), (4224, 160, 513), (4224, 416, 640), (4160, 96, 300),
-                                   (17920, 96, 65), (17920, 32, 333)])
+                                   (17920, 96, 65), (17920, 32, 333), (17920, 288, 77), (17920, 416, 200), (17920, 288, 333),
+                                   (17920, 160, 1100), (17920, 416, 400)])
 def test_mmq_t32_store_and_resid(cuda, N, K, T):
     import torch
     wb, dw, xq, dx = problem(N, K, T, N + K + T)
@@ -158,7 +161,81 @@ def test_mmq_t32_swiglu_is_the_quantized_store(cuda, T):
     assert np.allclose(ds[..., 1], ds[..., 0] * oq.cpu().numpy().reshape(T, -1, 32).sum(2), rtol=2e-3, atol=1e-3)
 
 
+# 64 x 32 with four K waves, 128 x 64; of 17920 rows 256 x 32 (77 and 200 tokens), 128 x 128 (333 and 1100), 128 x 64 (400)
+@pytest.mark.parametrize("N,K,T", [(4224, 416, 300), (4224, 288, 448), (4224, 416, 577), (17920, 288, 77), (17920, 416, 200), (17920, 288, 333),
+                                   (17920, 416, 1100), (17920, 288, 400)])
+def test_mmq_t32_swiglu_is_the_quantized_product(cuda, N, K, T):
+    """SWIGLU_Q8 gives the Q8_1 rule of silu(g) u of the float64 sums: codes within one step, few of them off, and d equal
+    to the fp16 of their block maximum / 127 within the error of the hardware exp2 and reciprocal (about 2e-6 relative) and
+    the sums (below 1e-5 of a block's largest value)."""
+    import torch
+    wb, dw, xq, dx = problem(N, K, T, T)
+    W = QM.Q4Mat(wb, N, K, "cuda")
+    xq_d = torch.from_numpy(xq).cuda()
+    xds_d = torch.from_numpy(np.stack([dx, np.zeros_like(dx)], -1)).cuda()
+    oq = torch.zeros(T, N // 2, dtype=torch.int8, device=cuda)
+    ods = torch.zeros(T, N // 64, 2, dtype=torch.float16, device=cuda)
+    call("q355_mmq_q4_0_q8_1", ptr(W.qs), ptr(W.d), N, K, ptr(xq_d), ptr(xds_d), T, 7, None, None, ptr(oq), ptr(ods), None, None)
+    torch.cuda.synchronize()
+    # whole Q8_1 blocks (64 rows): every wave's place in the widest workgroup, and the last
+    blocks = np.r_[0:4, 65, N // 64 - 1]
+    rows = (blocks[:, None] * 64 + np.arange(64)).reshape(-1)
+    y, _ = reference(wb.reshape(N, -1, 18)[rows].reshape(-1, 18), dw[rows], xq, dx, len(rows), K, T)
+    g, u = y[:, 0::2], y[:, 1::2]
+    with np.errstate(over="ignore"):
+        m = g / (1 + np.exp(-g)) * u
+    q, d, _ = OQ.quantize_q8_1(m.astype(np.float32))
+    got = oq.cpu().numpy().reshape(T, -1, 32)[:, blocks].reshape(T, -1)
+    dq = np.abs(got.astype(int) - q)
+    assert dq.max() <= 1 and (dq > 0).mean() < 1e-3
+    ds = ods.cpu().numpy().astype(np.float64)[:, blocks]
+    assert (np.abs(ds[..., 0] - d) <= 2.0 ** -10 * np.abs(d) + 2.0 ** -24).all()
+    assert np.allclose(ds[..., 1], ds[..., 0] * got.reshape(T, -1, 32).sum(2), rtol=2e-3, atol=1e-3)
+
+
 @pytest.mark.parametrize("T,seq_stride", [(33, 0), (64, 1), (65, 0), (255, 0), (256, 0), (511, 0), (512, 0)])
 def test_qkv_rope_forms(cuda, T, seq_stride):
     """The fused QKV finish of every form (k_mmq_s32 in f64 and fp32, four K waves, one) against the split product."""
     qkv_rope_equals_finish(cuda, T, seq_stride)
+
+
+# register-resident; k_mmq_s32 in f64 and fp32 (4, 12 and 16 slices); 64 x 64 below 256 tiles and from 512 tokens; four K
+# waves; 128 x 32; wide: 128 x 64, 128 x 128, 256 x 32
+@pytest.mark.parametrize("nh,nkv,K,T", [(12, 2, 512, 20), (12, 2, 512, 50), (12, 2, 1536, 40), (2, 1, 2048, 64),
+                                        (12, 2, 512, 255), (2, 1, 2048, 100), (12, 2, 480, 100), (28, 4, 288, 77),
+                                        (12, 2, 544, 300), (28, 4, 416, 300), (12, 2, 288, 520), (12, 2, 416, 1100),
+                                        (28, 4, 160, 600), (40, 8, 160, 1100), (50, 4, 160, 544)])
+def test_qkv_forms_against_float64(cuda, nh, nkv, K, T):
+    """q, K and V of every form of the fused QKV: the float64 product, bias and RoPE rounded to fp16 once, within the
+    products' fp32 bound."""
+    import torch
+    N, nq, nk = (nh + 2 * nkv) * 128, nh * 128, nkv * 128
+    wb, dw, xq, dx = problem(N, K, T, N + K + T)
+    W = QM.Q4Mat(wb, N, K, "cuda")
+    rng = np.random.default_rng(T)
+    bias = rng.standard_normal(N).astype(np.float32)
+    pages = (T + 63) // 64
+    table, pos = rng.permutation(pages).astype(np.int32), np.arange(T, dtype=np.int32)
+    cos, sin = QM.rope_tables(64 * pages)
+    t = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    kc = torch.zeros(pages, nkv, 64, 128, dtype=torch.float16, device=cuda)
+    vc = torch.zeros_like(kc)
+    q = torch.zeros(T, nq, dtype=torch.float16, device=cuda)
+    q64 = torch.zeros(T, nq, dtype=torch.float64, device=cuda)
+    args = [t(xq), t(np.stack([dx, np.zeros_like(dx)], -1)), t(bias), t(cos), t(sin), t(pos), t(table)]
+    p = [ptr(a) for a in args]
+    call("q355_mmq_qkv_rope", ptr(W.qs), ptr(W.d), N, K, p[0], p[1], T, *p[2:], pages, 0, ptr(kc), ptr(vc), ptr(q), ptr(q64),
+         nh, nkv)
+    torch.cuda.synchronize()
+    y, bound = reference(wb, dw, xq, dx, N, K, T)
+    y += bias.astype(np.float64)
+    a, b = (y[:, :nq + nk].reshape(T, nh + nkv, 64, 2)[..., i] for i in (0, 1))         # device rows: pairs (d, d + 64)
+    ea, eb = (bound[:, :nq + nk].reshape(T, nh + nkv, 64, 2)[..., i] for i in (0, 1))
+    c, s = (f[pos][:, None].astype(np.float64) for f in (cos, sin))
+    rot = np.concatenate([a * c - b * s, b * c + a * s], -1).reshape(T, -1)
+    tol = np.concatenate([ea * np.abs(c) + eb * np.abs(s), eb * np.abs(c) + ea * np.abs(s)], -1).reshape(T, -1)
+    rows = lambda x: x[table.astype(np.int64)].permute(0, 2, 1, 3).reshape(64 * pages, nk)[:T].cpu().numpy()  # noqa: E731
+    got = np.concatenate([q.cpu().numpy(), rows(kc), rows(vc)], 1).astype(np.float64)
+    want, tol = np.concatenate([rot, y[:, nq + nk:]], 1), np.concatenate([tol, bound[:, nq + nk:]], 1)
+    assert (np.abs(got - want) <= tol + 2.0 ** -11 * (np.abs(want) + tol) + 2.0 ** -25).all()
+    assert np.array_equal(q64.cpu().numpy(), got[:, :nq])
