@@ -522,7 +522,8 @@ static int launch_mmq_t32(const GemvArgs& a, hipStream_t s) {
 // From 512 tokens a wave takes the whole K, whatever T is, so that a prompt prefilled in chunks of 512 tokens and more
 // gives the sums of one chunk: up to two 64 x 64 workgroups per CU with chunks of 8 blocks (the wait for the next chunk is
 // what bounds them), more of them 128 x 32 with chunks of 4. us at 512 / 1024 / 2048 tokens, 1536 x 8960: 53 / 74 / 102
-// (the other form 59 / 77 / 114; 16x16x32 tiles 89 / 110 / 135); 1536 x 1536: 13.7 / 19.1 / 25; 2048 x 1536: 14.0 / 20.0 / 28.
+// (the other form 59 / 77 / 114; 16x16x32 tiles 89 / 110 / 135); 1536 x 1536: 13.7 / 19.1 / 25; 2048 x 1536 as a residual
+// 14.0 / 20.0 / 28, as the fused QKV 36 at 2048.
 // 256 to 511 tokens, and N % 128 == 64 from 256 on, have four chains over K (k_mmq<4> had them): four K waves per tile,
 // chunks of 8 (333 tokens: 1536 x 8960 35 us, 44 with chunks of 4, 89 for k_mmq<4>; 1536 x 1536 9.7, 11.5 and 19.8).
 template <int EPI>
@@ -537,6 +538,8 @@ static int launch_mmq_narrow(const GemvArgs& a, hipStream_t s) {
 // Prefill sizes (STORE, RESID_FIX, SWIGLU_Q8, QKV): k_mmq_t32. Wide matrices take one wave per tile, so the summation
 // order is the same whatever the workgroup: 256 x 32, 128 x 64 or 128 x 128, by what the fullest CU costs (us for c
 // workgroups on it, from 17920 x 1536: 256 x 32 20 + 8 (c - 1), 128 x 64 18 + 7.2 (c - 1), 128 x 128 28 + 11 (c - 1)).
+// The fixed parts do not grow with K as the others do, but the choice held: over 4224 to 17920 rows, K 1536 to 6144 and 512 to
+// 2048 tokens it was within 3 % of the best of the three, once (17920 x 1536 at 1024 tokens) 7 % off.
 // 17920 x 1536 (us; 16x16x32 tiles before): 77 tokens 20.3 (23.5), 200: 28 (34), 333: 39 (57), 2048: 160 (213).
 // Fewer than 256 tiles of 128 x 64 below 512 tokens: the narrow forms, whatever the width. From 256 tokens these keep four
 // chains over K (one would double the error: 4608 x 3584 at 300 tokens 1.9e-7 against 1.0e-7; k_mmq<4> 75 us, one wave per
@@ -573,8 +576,7 @@ static int launch_mmq_logits_tile(const GemvArgs& a, hipStream_t s) {
   if (a.T > 16)
     return a.N / 128 <= 2 * device_cus() ? launch_mmq_t32<2, 1, 1, 1, 1, 8, EPI_LOGITS>(a, s)
                                          : launch_mmq_t32<2, 1, 2, 1, 1, 4, EPI_LOGITS>(a, s);
-  constexpr size_t lds = 2 * LdsTile<2, TILE_CB>::BUF;
-  hipLaunchKernelGGL(k_mmq_tile<2>, dim3(a.N / 128, 1, 1), dim3(128), lds, s, a);
+  hipLaunchKernelGGL(k_mmq_tile, dim3(a.N / (TILE_RW * 64), 1, 1), dim3(TILE_RW * 64), 2 * LdsTile::BUF, s, a);
   return launched("mmq");
 }
 

@@ -573,18 +573,19 @@ __global__ void __launch_bounds__(NW * 64) k_mmq_reg(const GemvArgs a) {
 //   X  [CB][16]                            activation scale / 16 (fp32)
 // Epilogue from registers: fp32 logits and one (max, row) partial per 64 rows and token, the layout of the other LOGITS
 // kernels.
-template <int RW, int CB>
+constexpr int TILE_RW = 2;                           // waves per workgroup
+
 struct LdsTile {
+  static constexpr int RW = TILE_RW, CB = TILE_CB;
   static constexpr int TW = 16;                      // tokens per workgroup
   static constexpr int A = RW * 4 * CB * 256, W = RW * 4 * CB * 64, B = CB * 512;
   static constexpr int X = CB * TW * 4;
   static constexpr int BUF = A + W + B + X;
 };
 
-template <int RW>
-__global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
-  constexpr int CB = TILE_CB;
-  using L = LdsTile<RW, CB>;
+__global__ void __launch_bounds__(TILE_RW * 64) k_mmq_tile(const GemvArgs a) {
+  using L = LdsTile;
+  constexpr int RW = L::RW, CB = L::CB;
   constexpr int TW = L::TW;
   constexpr int NTH = RW * 64;                       // threads
   constexpr int NA = RW * 4 * CB * 16;               // 16-byte pieces of A per chunk
@@ -725,8 +726,9 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
 }
 
 // Prefill-size GEMM on v_mfma_i32_32x32x32_i8: a workgroup computes RW x CW wave tiles of (32 RT rows) x (32 TN
-// tokens) over the whole K. KW waves share a tile: each takes every KW-th K block, and their fp32 sums are added in f64
-// in the order of the waves. So a result depends on KW but not on the tile's or the workgroup's shape.
+// tokens) over the whole K. KW waves share a tile: each takes every KW-th block of a chunk of CB (a partial last chunk starts
+// CB blocks before the end of K, so there a block's wave is by its place from the end), and their fp32 sums are added in f64
+// in the order of the waves. So a result depends on KW, and with KW > 1 on CB, but not on the tile's or the workgroup's shape.
 // One 32-row tile of one Q4_0 block against 32 tokens is one MFMA. Lane l holds A[row l % 32][k = 16 (l / 32) .. +16]:
 // the low (lanes 0..31) or high nibbles of the row's 16 bytes as int8 16 (q - 8); B[k = 16 (l / 32) .. +16][token
 // l % 32]; and C[row 8 (v / 4) + 4 (l / 32) + v % 4][token l % 32], v = 0 .. 15. The d_w d_x of a tile come from one
@@ -736,7 +738,7 @@ __global__ void __launch_bounds__(256) k_mmq_tile(const GemvArgs a) {
 // What bounds it: VALU issue. A 32 x 32 tile and block needs 16 int32 -> fp32 converts and 16 fmas (each about 4.3
 // cycles of a SIMD while the matrix cores run), against 64 cycles of int8 and fp16 MFMAs that run beside them; the
 // unpacking, staging and epilogue add 15 more VALU instructions. fp32 scale products (v_mfma_f32_32x32x1) would hold
-// the VALU up: converts do not overlap with them. Counters at 17920 x 1536 x 2048 tokens: VALU 84 % busy.
+// the VALU up: converts do not overlap with them. Counters at 17920 x 1536 x 2048 tokens: VALU 86 % busy.
 // Measured (us, 2048 tokens; before: 16x16x32 products with fp32 scale products): 17920 x 1536 213 -> 160 in 128 x 128
 // workgroups (174 in 128 x 64), 1536 x 8960 135 -> 102, 1536 x 1536 32 -> 25 and 2048 x 1536 34 -> 28 in 128 x 32 ones of
 // a 32 x 32 tile per wave. The tied head (151936 x 1536, LOGITS) at 24 and 32 tokens 43 -> 36 in 128 x 32 workgroups of two

@@ -334,7 +334,8 @@ class Prefill:
         self.h = torch.zeros(P, H, dtype=torch.int64, device=dev)
         self.xq = torch.zeros(P, max(H, c.FFN), dtype=torch.int8, device=dev)
         self.xds = torch.zeros(P, max(H, c.FFN) // 32, 2, dtype=torch.float16, device=dev)
-        self.qkv_acc = torch.zeros(P, c.nqkv, dtype=torch.int64, device=dev)
+        split = min(P, QKV_FUSED_MIN_P - 1)                # the longest chunk whose QKV product is not fused, if any
+        self.qkv_acc = torch.zeros(split, c.nqkv, dtype=torch.int64, device=dev) if split > self.qkv_small_p else None
         self.q = torch.zeros(P, c.NH * c.HD, dtype=torch.float16, device=dev)
         self.mq = torch.zeros(P, c.FFN, dtype=torch.int8, device=dev)
         self.mds = torch.zeros(P, c.FFN // 32, 2, dtype=torch.float16, device=dev)
