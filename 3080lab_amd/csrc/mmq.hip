@@ -1091,9 +1091,9 @@ __global__ void __launch_bounds__(RW * CW * KW * 64) k_mmq_t32(const GemvArgs a)
 // per output and slice) had been most of the time. QKV adds the slices, rounded to the same 2^-48, in f64: the same sums
 // where the fixed point holds them (|sum| < 2^15), and large, infinite and NaN ones stay what they are.
 // A wave loads the blocks of two slices before its first product: one memory latency.
-// Measured (us at 77 / 150 / 250 tokens; k_mmq_reg with atomics before): 1536 x 1536 9.6 / 9.9 / 17.2 (11.8 / 20 / 31), 2048 x
-// 1536 9.8 / 16.5 / 17.7 (16.5 / 24 / 38). Bounded by two memory latencies and the f64 rounding; past one workgroup per
-// CU (registers) by their rounds.
+// Measured (us at 77 / 150 / 250 tokens; k_mmq_reg with atomics before): RESID_FIX of 1536 x 1536 9.6 / 9.9 / 17.2 (11.8 / 20 /
+// 31); QKV of 2048 x 1536 at 77 / 128 / 200 / 255 tokens 8.9 / 9.1 / 16.4 / 16.6 (the split product alone 16.5 / 21 / 31 / 38).
+// Bounded by two memory latencies and the f64 rounding; past one workgroup per CU (registers) by their rounds.
 constexpr int S32_KW = 6;
 
 template <int EPI, bool F64>

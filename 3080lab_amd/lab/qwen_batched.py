@@ -302,8 +302,8 @@ def flash_prefill_v3_source(maxlen: int = 4096, q8: bool = True) -> KernelSpec:
 
 
 # chunks of at least this many tokens, and short ones, run the QKV product with the finish in its epilogue
-# (q355_mmq_qkv_rope: one launch, no int64 accumulator; 2048 x 1536 at 77 tokens: 10 us against 16.5 + 5.4, at 333 tokens:
-# 12 against 24 + 6). Short is what the library says it sums as precisely as the split form (qkv_fused_small_p). The others
+# (q355_mmq_qkv_rope: one launch, no int64 accumulator; 2048 x 1536 at 77 tokens: 9 us against 16.5 + 5.4, at 333 tokens: 12
+# against 24 + 6). Short is what the library says it sums as precisely as the split form (qkv_fused_small_p). The others
 # keep the K-split product into the int64 accumulator plus q355_qkv_finish. From 512 tokens on no product's summation
 # order depends on the chunk, so chunking a prompt into pieces of >= 512 tokens gives the same results bit for bit.
 QKV_FUSED_MIN_P = 256
